@@ -233,3 +233,67 @@ def work(case):
 
 def tolerance(case):
     return {"rel": _REL[case["dtype"]]}
+
+
+def _taps(x, front, weight, bias, ids):
+    """SiLU of the causal convolution of x (batch, dim, seqlen) behind `front` (batch, dim, width-1), as
+    shifted products in the type of x; a tap counts where its position has the id of the output's."""
+    width, seqlen = weight.shape[1], x.shape[2]
+    padded = torch.cat([front, x], dim=2)
+    if ids is not None:
+        ids = torch.nn.functional.pad(ids, (width - 1, 0), value=-1)
+    acc = bias.view(1, -1, 1).expand_as(x)
+    for w in range(width):
+        term = padded[:, :, w:w + seqlen] * weight[:, w].view(1, -1, 1)
+        if ids is not None:
+            term = torch.where((ids[:, w:w + seqlen] == ids[:, width - 1:]).unsqueeze(1), term, 0.0)
+        acc = acc + term
+    return acc * torch.sigmoid(acc)
+
+
+def _decode_layer(x, cache, weight, bias, lengths, indices):
+    width, state_len = weight.shape[1], cache.shape[2]
+    new = (x.unsqueeze(2) if x.dim() == 2 else x).double()
+    rows = torch.arange(new.shape[0], device=x.device) if indices is None else indices.long()
+    live = rows >= 0
+    old = cache[rows.clamp(min=0)]
+    if lengths is None:
+        window = old[:, :, state_len - (width - 1):]
+        kept = torch.cat([old, new], dim=2)[:, :, -state_len:]
+    else:
+        at = torch.arange(-(width - 1), new.shape[2], device=x.device) + lengths.long().view(-1, 1)
+        at = (at % state_len).unsqueeze(1).expand(-1, new.shape[1], -1)
+        window = old.gather(2, at[..., :width - 1])
+        kept = old.scatter(2, at[..., width - 1:], new)
+    cache[rows[live]] = kept[live]
+    out = torch.where(live.view(-1, 1, 1), _taps(new, window, weight.double(), bias.double(), None), 0.0)
+    return out.squeeze(2) if x.dim() == 2 else out
+
+
+def exact(case, seed):
+    """What `run` returns for these inputs, in 64 bits and plain torch."""
+    s = prepare(case, seed)
+    if s["path"] == "decode":
+        caches = s["all_caches"].double()
+        outs = [_decode_layer(x, cache, weight, bias, s["lengths"], s["indices"])
+                for x, cache, weight, bias in zip(s["xs"], caches.unbind(0), s["weights"], s["biases"])]
+        return {"outs": outs, "caches": caches}
+    leaves = [s[k].detach().double().requires_grad_(s["path"] == "train") for k in ("x", "weight", "bias")]
+    x, weight, bias = leaves
+    front = torch.zeros_like(x[:, :, :weight.shape[1] - 1])
+    if s.get("init") is not None:
+        front = s["init"].detach().double().requires_grad_(s["path"] == "train")
+        leaves.append(front)
+    out = _taps(x, front, weight, bias, s["ids"])
+    if s["path"] == "handoff":
+        n, cu = s["state_len"], s["cu"].tolist()
+        states = x.new_zeros(len(cu) - 1, x.shape[1], n)
+        for b, (lo, hi) in enumerate(zip(cu, cu[1:])):
+            k = min(n, hi - lo)
+            states[b, :, n - k:] = x[0, :, hi - k:hi]
+        return out, states
+    outs = [out] if s.get("init") is None else [out, x[:, :, 1 - weight.shape[1]:]]
+    if s["path"] == "prefill":
+        return outs[0] if len(outs) == 1 else tuple(outs)
+    grads = torch.autograd.grad(outs, leaves, [g.double() for g in s["grads"]])
+    return {"outs": [t.detach() for t in outs], "grads": grads}
