@@ -386,6 +386,40 @@ struct StridedTaps {
     }
 };
 
+// Taps and bias of one channel as fp32, any strides and type.  One branch on the type for all of them:
+// with a branch per element each load waits for everything in flight before the next is issued, five
+// waits in a row.  Taps of 16 bits, bf16 data, channel-first: backward (16, 4096, 1001) 116 -> 82 us,
+// see cc1d_fwd_channelfirst_tile.hip for the forward.
+template <int W>
+__device__ __forceinline__ void channel_taps(const void *weight, const void *bias, int w_dtype, int64_t stride_c,
+                                             int64_t stride_w, int c, float (&wv)[W], float &bv) {
+    if (w_dtype == CC1D_F32) {
+        const float *wp = reinterpret_cast<const float *>(weight) + (int64_t)c * stride_c;
+#pragma unroll
+        for (int w = 0; w < W; ++w) wv[w] = wp[(int64_t)w * stride_w];
+        bv = bias != nullptr ? reinterpret_cast<const float *>(bias)[c] : 0.f;
+    } else {
+        uint16_t raw[W + 1];
+        const uint16_t *wp = reinterpret_cast<const uint16_t *>(weight) + (int64_t)c * stride_c;
+#pragma unroll
+        for (int w = 0; w < W; ++w) raw[w] = wp[(int64_t)w * stride_w];
+        raw[W] = bias != nullptr ? reinterpret_cast<const uint16_t *>(bias)[c] : (uint16_t)0;
+        const bool bf16 = w_dtype == CC1D_BF16;
+#pragma unroll
+        for (int w = 0; w < W; ++w) wv[w] = bf16 ? bitcast<float>((uint32_t)raw[w] << 16) : (float)bitcast<_Float16>(raw[w]);
+        bv = bf16 ? bitcast<float>((uint32_t)raw[W] << 16) : (float)bitcast<_Float16>(raw[W]);
+    }
+}
+// The same for a channel that all lanes of the wavefront share: the values end in scalar registers.
+template <int W>
+__device__ __forceinline__ void uniform_taps(const void *weight, const void *bias, int w_dtype, int64_t stride_c,
+                                             int64_t stride_w, int c, float (&wv)[W], float &bv) {
+    channel_taps<W>(weight, bias, w_dtype, stride_c, stride_w, c, wv, bv);
+#pragma unroll
+    for (int w = 0; w < W; ++w) wv[w] = bitcast<float>(__builtin_amdgcn_readfirstlane(bitcast<int>(wv[w])));
+    bv = bitcast<float>(__builtin_amdgcn_readfirstlane(bitcast<int>(bv)));
+}
+
 // ---------------------------------------------------------------------------------
 // Wave64 lane shifts through DPP (no LDS, no memory).  All 64 lanes must be active.
 //   from_prev_lane: lane i receives lane i-1's value, lane 0 receives `lane0_fill`.

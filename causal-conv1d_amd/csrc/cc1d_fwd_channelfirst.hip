@@ -122,10 +122,7 @@ fwd_channelfirst_kernel(const cc1d_fwd_params p, const FwdCfGeom g) {
 
     if (j_begin < j_end) {
         float wv[W], bias_v;
-#pragma unroll
-        for (int w = 0; w < W; ++w)
-            wv[w] = ld_weight(p.weight, p.w_dtype, (int64_t)c * p.w_stride_c + w * p.w_stride_w);
-        bias_v = p.bias == nullptr ? 0.f : ld_weight(p.bias, p.w_dtype, c);
+        channel_taps<W>(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, c, wv, bias_v);
         // The arithmetic of the other kernels, bit for bit: taps and bias carry the factor
         // -log2(e) where the activation takes the sums as its exponent (see silu_from_scaled).
         const bool scaled = silu_on && !PRECISE;
@@ -261,10 +258,7 @@ fwd_channelfirst_stream_kernel(const cc1d_fwd_params p, const FwdCfGeom g) {
     const int n_groups = n_full > 0 ? n_full / (2 * U) * 2 : 0;
 
     float wv[W], bias_v;
-#pragma unroll
-    for (int w = 0; w < W; ++w)
-        wv[w] = ld_weight(p.weight, p.w_dtype, (int64_t)c * p.w_stride_c + w * p.w_stride_w);
-    bias_v = p.bias == nullptr ? 0.f : ld_weight(p.bias, p.w_dtype, c);
+    channel_taps<W>(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, c, wv, bias_v);
     if (SCALED) {
         bias_v *= kSiluPrescale;
 #pragma unroll
@@ -492,10 +486,7 @@ fwd_channelfirst_short_kernel(const cc1d_fwd_params p, const int n_vecs, const i
         __builtin_memcpy(&raw, elems, sizeof raw);
     }
     float wv[W], bias_v;
-#pragma unroll
-    for (int w = 0; w < W; ++w)
-        wv[w] = ld_weight(p.weight, p.w_dtype, (int64_t)c * p.w_stride_c + w * p.w_stride_w);
-    bias_v = p.bias == nullptr ? 0.f : ld_weight(p.bias, p.w_dtype, c);
+    channel_taps<W>(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, c, wv, bias_v);
     float halo[W - 1];
 #pragma unroll
     for (int i = 0; i < W - 1; ++i) halo[i] = 0.f;
@@ -637,26 +628,21 @@ fwd_channelfirst_flat_kernel(const cc1d_fwd_params p, const uint32_t n_elems) {
     // (one lane in seqlen / VEC).  Packed fp32 taps (a host-checked promise: strides (W, 1), base
     // 16-byte aligned) of even width come in one load.
     float w0[W], w1[W], bias0, bias1 = 0.f;
-    auto taps = [&](uint32_t c, float (&wv)[W]) {
+    auto taps = [&](uint32_t c, float (&wv)[W], float &bv) {
         if (PACKED_W && W % 2 == 0) {
             const float *src = static_cast<const float *>(__builtin_assume_aligned(
                 reinterpret_cast<const float *>(p.weight) + (int64_t)c * W, W % 2 == 0 ? W * 4 : 4));
 #pragma unroll
             for (int w = 0; w < W; ++w) wv[w] = src[w];
+            bv = p.bias == nullptr ? 0.f : reinterpret_cast<const float *>(p.bias)[c];   // of the taps' type
         } else {
-#pragma unroll
-            for (int w = 0; w < W; ++w)
-                wv[w] = ld_weight(p.weight, p.w_dtype, (int64_t)c * p.w_stride_c + w * p.w_stride_w);
+            channel_taps<W>(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, (int)c, wv, bv);
         }
     };
-    taps(c0, w0);
-    bias0 = p.bias == nullptr ? 0.f : ld_weight(p.bias, p.w_dtype, c0);
+    taps(c0, w0, bias0);
 #pragma unroll
     for (int w = 0; w < W; ++w) w1[w] = 0.f;
-    if (split < (uint32_t)VEC) {
-        taps(c1, w1);
-        bias1 = p.bias == nullptr ? 0.f : ld_weight(p.bias, p.w_dtype, c1);
-    }
+    if (split < (uint32_t)VEC) taps(c1, w1, bias1);
     if (SCALED) {
         bias0 *= kSiluPrescale;
         bias1 *= kSiluPrescale;
