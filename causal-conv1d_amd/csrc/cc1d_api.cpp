@@ -306,6 +306,7 @@ Knob *find_knob(const char *name) {
         {"bwd_cl_lane_bytes", &Tunables::bwd_cl_lane_bytes},
         {"fwd_cf_vecs", &Tunables::fwd_cf_vecs},
         {"bwd_cf_parts", &Tunables::bwd_cf_parts},
+        {"bwd_cf_direct", &Tunables::bwd_cf_direct},
         {"launch_limit_shift", &Tunables::launch_limit_shift},
     };
     for (const auto &e : table)

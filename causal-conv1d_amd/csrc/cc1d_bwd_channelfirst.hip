@@ -175,10 +175,7 @@ bwd_channelfirst_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float *__res
     RowCtx<DT, W> rc{p};
     rc.c = c;
     rc.silu_on = p.silu != 0;
-#pragma unroll
-    for (int w = 0; w < W; ++w)
-        rc.wv[w] = ld_weight(p.weight, p.w_dtype, (int64_t)c * p.w_stride_c + w * p.w_stride_w);
-    rc.bias_v = p.bias == nullptr ? 0.f : ld_weight(p.bias, p.w_dtype, c);
+    channel_taps<W>(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, c, rc.wv, rc.bias_v);
     rc.scale_taps();
 
     float dW[W], dB = 0.f;
@@ -391,10 +388,7 @@ bwd_channelfirst_stream_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float
     RowCtx<DT, W> rc{p};
     rc.c = c;
     rc.silu_on = p.silu != 0;
-#pragma unroll
-    for (int w = 0; w < W; ++w)
-        rc.wv[w] = ld_weight(p.weight, p.w_dtype, (int64_t)c * p.w_stride_c + w * p.w_stride_w);
-    rc.bias_v = p.bias == nullptr ? 0.f : ld_weight(p.bias, p.w_dtype, c);
+    channel_taps<W>(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, c, rc.wv, rc.bias_v);
     rc.scale_taps();
 
     float dW[W], dB = 0.f;
@@ -692,10 +686,7 @@ bwd_channelfirst_short_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float 
     const bool silu_on = p.silu != 0;
 
     float wv[W], bias_v;
-#pragma unroll
-    for (int w = 0; w < W; ++w)
-        wv[w] = ld_weight(p.weight, p.w_dtype, (int64_t)c * p.w_stride_c + w * p.w_stride_w);
-    bias_v = p.bias == nullptr ? 0.f : ld_weight(p.bias, p.w_dtype, c);
+    channel_taps<W>(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, c, wv, bias_v);
     float wvs[W];
 #pragma unroll
     for (int w = 0; w < W; ++w) wvs[w] = wv[w] * kSiluPrescale;
@@ -1000,7 +991,7 @@ int launch_bwd_channelfirst(const cc1d_bwd_params &p, void *workspace, hipStream
     float *ws = static_cast<float *>(workspace);
     if (takes_tiles(p)) {
         const int st = launch_bwd_channelfirst_tile(p, ws, stream);
-        if (st != CC1D_OK) return st;
+        if (st != CC1D_OK || bwd_channelfirst_tile_direct(p)) return st;   // the kernel wrote dweight / dbias itself
         return launch_bwd_finalize(ws, bwd_channelfirst_tile_parts(p), p, stream);
     }
     const BwdCfGeom g = make_geom(p);

@@ -33,9 +33,9 @@
 // vector in LDS; the g values to the right of its vector come from the next lane (DPP shift),
 // for the last lane from the step above (carried), for the top step from the vectors behind the
 // tile.  The lane's dweight / dbias terms stay in registers across the tile, are reduced over
-// the 64 lanes in a fixed order (DPP) and stored as one workspace plane per (batch entry, tile);
-// the second-stage kernel shared with the other backward kernels adds the planes in a fixed
-// order: no atomics, bit-reproducible.
+// the 64 lanes in a fixed order (DPP) and either stored as one workspace plane per (batch entry, tile),
+// which the second-stage kernel shared with the other backward kernels adds up in a fixed order, or,
+// where one workgroup holds all tiles of a channel, added up there: no atomics, bit-reproducible.
 #include <type_traits>
 
 #include "cc1d_device.hpp"
@@ -48,6 +48,7 @@ namespace {
 // with its taps, its g values behind the tile and its reduction (fp16 (4, 4096, 8192): three steps
 // 145 us, two 150 us against 140 us); six and eight measured no better than four.
 constexpr int kTileSteps = 4;
+constexpr int kMaxDirectTiles = 16;              // most tiles of a channel that one workgroup takes
 constexpr int kTailVecs = kWave / 4;              // most vectors 64 positions can span (fp32)
 constexpr int kRsrcRaw = 0x00020000;              // buffer resource word 3: raw buffer, 32-bit data format
 
@@ -68,7 +69,10 @@ struct BwdCfTileArgs {
     void *dx;
     const void *weight;
     const void *bias;
-    float *ws;                    // [batch * tiles_per_row][W + 1][dim]
+    float *ws;                    // [batch * tiles_per_row][W + 1][dim]; unused by DIRECT
+    float *dweight, *dbias;       // written by DIRECT
+    int64_t dw_stride_c, dw_stride_w;
+    int32_t overwrite;
     int64_t x_stride_b, x_stride_c, dout_stride_b, dout_stride_c, dx_stride_b, dx_stride_c;   // elements
     int64_t w_stride_c, w_stride_w;
     const void *initial_states;
@@ -91,8 +95,18 @@ __device__ __forceinline__ float wave_total_in_lane63(float v) {
     return v;
 }
 
-template <int DT, int W, bool SILU>
-__global__ void __launch_bounds__(kBlock, 4)
+// DIRECT: a workgroup is one channel and its wavefronts are the channel's tiles, so that it can add up
+// their sums itself and store dweight / dbias: one launch instead of two, and no workspace
+// traffic.  Otherwise the wavefronts are numbered along the rows, four to a workgroup, and leave their
+// sums to the second stage.  See tile_sums_directly for the line between the two.
+// Registers: 64 at most (16-bit data), so that eight wavefronts share a SIMD; wave-uniform values
+// (taps, the odd last element, dfinal_states) live in scalar registers for that.  The launch is bound
+// by memory and by the vector ALUs about equally, and what counts is how well the two overlap:
+// 65 registers and seven wavefronts measured (16, 4096, 1001) bf16 85.0 us against 80.8 now with 57
+// and eight, (16, 4096, 1024) 75.6 against 73.3, fp16 (4, 4096, 8192) 139.2 against 136.2 (second stage
+// included).
+template <int DT, int W, bool SILU, bool DIRECT>
+__global__ void __launch_bounds__(DIRECT ? kMaxDirectTiles * kWave : kBlock, 4)
 bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
     using E = Elem<DT>;
     using T = typename E::type;
@@ -105,12 +119,13 @@ bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
 
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const int lane = (int)(threadIdx.x & (kWave - 1));
-    const uint32_t wid = blockIdx.x * (uint32_t)(kBlock / kWave) + (uint32_t)wv;
-    if (wid >= a.total) return;
+    const uint32_t wid = DIRECT ? (uint32_t)wv : blockIdx.x * (uint32_t)(kBlock / kWave) + (uint32_t)wv;
+    if (!DIRECT && wid >= a.total) return;
     const int tile = (int)(wid % a.tiles_per_row);
-    const uint32_t row = wid / a.tiles_per_row;
+    const uint32_t row = wid / a.tiles_per_row;       // DIRECT: of the channel's rows
     int b, c;
-    if (a.batch_inner) { b = (int)(row % (uint32_t)a.batch); c = (int)(row / (uint32_t)a.batch); }
+    if (DIRECT) { b = (int)row; c = (int)blockIdx.x; }
+    else if (a.batch_inner) { b = (int)(row % (uint32_t)a.batch); c = (int)(row / (uint32_t)a.batch); }
     else { c = (int)(row % (uint32_t)a.dim); b = (int)(row / (uint32_t)a.dim); }
     const int L = a.seqlen;
 
@@ -170,10 +185,7 @@ bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
     // Taps and bias of the channel (wave-uniform); with the fast activation also times -log2(e),
     // so that the sum over the window is the exponent the derivative needs.
     float wv_[W], wvs[W], bias_v, bias_s;
-#pragma unroll
-    for (int w = 0; w < W; ++w)
-        wv_[w] = ld_weight(a.weight, a.w_dtype, (int64_t)c * a.w_stride_c + w * a.w_stride_w);
-    bias_v = a.bias == nullptr ? 0.f : ld_weight(a.bias, a.w_dtype, c);
+    uniform_taps<W>(a.weight, a.bias, a.w_dtype, a.w_stride_c, a.w_stride_w, c, wv_, bias_v);
 #pragma unroll
     for (int w = 0; w < W; ++w) wvs[w] = wv_[w] * kSiluPrescale;
     bias_s = bias_v * kSiluPrescale;
@@ -210,6 +222,10 @@ bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
     // Every vector of the tile is in LDS behind this wait (a vector fetched into LDS counts as a
     // load until it has been written there).
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // wave-uniform values to scalar registers
+#pragma unroll
+    for (int i = 0; i < W - 1; ++i) dfin[i] = bitcast<float>(__builtin_amdgcn_readfirstlane(bitcast<int>(dfin[i])));
+    const float last_dout = bitcast<float>(__builtin_amdgcn_readfirstlane(bitcast<int>(E::to_float(last_d))));
     if (holds_last && lane == 0) {
         // LDS element index of row position p: p + VEC - tile_first
         const int ix = L - 1 + VEC - tile_first;
@@ -255,6 +271,10 @@ bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
         for (int k = 0; k < W; ++k) dW[k] = fmaf(g[0], xw[k], dW[k]);
 #pragma unroll
         for (int e = 0; e < W - 1; ++e) carry[e] = read_lane(g[0], e);
+    } else if (tile_end >= L) {
+        // the row ends with the tile: no g behind it
+#pragma unroll
+        for (int e = 0; e < W - 1; ++e) carry[e] = 0.f;
     } else {
         float xa[VEC], xb[VEC], dv[VEC];
         E::unpack(xl[steps * kWave], xa);
@@ -278,7 +298,7 @@ bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
         const int step_first = (v0 + s * kWave) * VEC;
         if (holds_last && L - 1 >= step_first && L - 1 < step_first + kWave * VEC) {
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) dv[e] = p0 + e == L - 1 ? E::to_float(last_d) : dv[e];
+            for (int e = 0; e < VEC; ++e) dv[e] = p0 + e == L - 1 ? last_dout : dv[e];
         }
         // xw[i] = padded x at position (first position of the lane's vector) - (W-1) + i
         float xw[VEC + W - 1], g[VEC + W - 1];
@@ -336,6 +356,25 @@ bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
 #pragma unroll
     for (int w = 0; w < W; ++w) dW[w] = wave_total_in_lane63(dW[w]);
     dB = wave_total_in_lane63(dB);
+    if constexpr (DIRECT) {
+        // The channel's tiles are this workgroup's wavefronts: their sums are added in order and stored.
+        const int waves = (int)(blockDim.x / kWave);
+        float *sums = reinterpret_cast<float *>(lds + waves * XV);
+        if (lane == kWave - 1) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) sums[wv * (W + 1) + w] = dW[w];
+            sums[wv * (W + 1) + W] = dB;
+        }
+        __syncthreads();
+        const int w = (int)threadIdx.x;
+        if (w < W || (w == W && a.dbias != nullptr)) {
+            float total = 0.f;
+            for (int i = 0; i < waves; ++i) total += sums[i * (W + 1) + w];
+            float *dst = w < W ? a.dweight + (int64_t)c * a.dw_stride_c + (int64_t)w * a.dw_stride_w : a.dbias + c;
+            *dst = a.overwrite ? total : *dst + total;
+        }
+        return;
+    }
     if (lane == kWave - 1) {
         float *dst = a.ws + ((int64_t)b * a.tiles_per_row + tile) * (int64_t)(W + 1) * a.dim + c;
 #pragma unroll
@@ -344,22 +383,28 @@ bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
     }
 }
 
-template <int DT, int W>
+// LDS of one wavefront: steps_per_tile steps of x, the vectors around them, room for a tail, its sums.
+size_t tile_lds_bytes(int steps, int width) {
+    return (size_t)(steps * kWave + 2 + kTailVecs) * sizeof(u32x4) + (size_t)(width + 1) * sizeof(float);
+}
+
+template <int DT, int W, bool DIRECT>
 int launch_tile_act(const cc1d_bwd_params &p, const BwdCfTileArgs &a, hipStream_t stream) {
-    const uint32_t blocks = (a.total + (kBlock / kWave) - 1) / (kBlock / kWave);
-    // per wavefront: steps_per_tile steps of x, the vectors around them, room for a tail
-    const size_t lds = (size_t)(kBlock / kWave) * (a.steps_per_tile * kWave + 2 + kTailVecs) * sizeof(u32x4);
-    if (p.silu) CC1D_LAUNCH((bwd_channelfirst_tile_kernel<DT, W, true>), dim3(blocks), dim3(kBlock), lds, stream, a);
-    else CC1D_LAUNCH((bwd_channelfirst_tile_kernel<DT, W, false>), dim3(blocks), dim3(kBlock), lds, stream, a);
+    const uint32_t waves = DIRECT ? (uint32_t)bwd_channelfirst_tile_parts(p) : (uint32_t)(kBlock / kWave);
+    const uint32_t blocks = DIRECT ? (uint32_t)p.dim : (a.total + waves - 1) / waves;
+    const size_t lds = waves * tile_lds_bytes(a.steps_per_tile, W);
+    if (p.silu) CC1D_LAUNCH((bwd_channelfirst_tile_kernel<DT, W, true, DIRECT>), dim3(blocks), dim3(waves * kWave), lds, stream, a);
+    else CC1D_LAUNCH((bwd_channelfirst_tile_kernel<DT, W, false, DIRECT>), dim3(blocks), dim3(waves * kWave), lds, stream, a);
     return launch_status();
 }
 
 template <int DT>
 int launch_tile_width(const cc1d_bwd_params &p, const BwdCfTileArgs &a, hipStream_t stream) {
+    const bool direct = bwd_channelfirst_tile_direct(p);
     switch (p.width) {
-        case 2: return launch_tile_act<DT, 2>(p, a, stream);
-        case 3: return launch_tile_act<DT, 3>(p, a, stream);
-        default: return launch_tile_act<DT, 4>(p, a, stream);
+        case 2: return direct ? launch_tile_act<DT, 2, true>(p, a, stream) : launch_tile_act<DT, 2, false>(p, a, stream);
+        case 3: return direct ? launch_tile_act<DT, 3, true>(p, a, stream) : launch_tile_act<DT, 3, false>(p, a, stream);
+        default: return direct ? launch_tile_act<DT, 4, true>(p, a, stream) : launch_tile_act<DT, 4, false>(p, a, stream);
     }
 }
 
@@ -396,6 +441,23 @@ bool bwd_channelfirst_tile_applies(const cc1d_bwd_params &p) {
 
 int bwd_channelfirst_tile_parts(const cc1d_bwd_params &p) { return (int)(p.batch * tiles_per_row(p)); }
 
+// Whether the kernel adds up the sums of a channel's tiles itself (DIRECT) instead of leaving them
+// to a second launch.  One workgroup must hold them all (its wavefronts, 64 KiB of LDS), and what the
+// second launch costs (2-3 us) must be more than what the other order of the tiles does: a
+// workgroup then reads and writes as many places as there are batch entries, where otherwise the launch
+// moves through memory as one front in the order of the rows.  Two places cost nothing; more of them
+// are worth it up to 8192 wavefronts.  Second stage / direct, us: (2, 64, 512) fp32 5.8 / 3.5,
+// (1, 5376, 2048) bf16 18.5 / 15.7, (1, 8192, 8192) 69.5 / 65.3, (2, 5376, 8192) fp16 88.9 / 86.8,
+// (8, 1024, 1024) bf16 15.2 / 13.2, (4, 2048, 1001) 16.1 / 15.4, (4, 2048, 2048) 23.1 / 23.3, and beyond the line
+// (4, 4096, 1001) 25.4 / 25.8, (8, 2048, 1024) 23.1 / 25.2, (4, 4096, 2048) 39.9 / 42.6.
+bool bwd_channelfirst_tile_direct(const cc1d_bwd_params &p) {
+    const int64_t tiles = (int64_t)p.batch * tiles_per_row(p);
+    if (tunables().bwd_cf_direct < 0 || tiles > kMaxDirectTiles || (size_t)tiles * tile_lds_bytes(steps_per_tile(p), p.width) > 64 * 1024)
+        return false;
+    const bool adjacent = p.batch <= 2 || (p.dim > 1 && p.x_stride_b < p.x_stride_c);   // a channel's rows lie together
+    return adjacent || (int64_t)p.dim * tiles <= 8192;
+}
+
 bool bwd_channelfirst_tile_fits(const cc1d_bwd_params &p) {
     return (int64_t)p.batch * p.dim * tiles_per_row(p) < wave_limit() && (int64_t)p.batch * tiles_per_row(p) < ((int64_t)1 << 30);
 }
@@ -404,6 +466,9 @@ int launch_bwd_channelfirst_tile(const cc1d_bwd_params &p, float *ws, hipStream_
     if (!bwd_channelfirst_tile_fits(p)) return CC1D_ERR_TOO_LARGE;
     BwdCfTileArgs a = {};
     a.tiles_per_row = (uint32_t)tiles_per_row(p);
+    a.dweight = p.dweight; a.dbias = p.dbias;
+    a.dw_stride_c = p.dw_stride_c; a.dw_stride_w = p.dw_stride_w;
+    a.overwrite = p.overwrite_dweight;
     a.steps_per_tile = steps_per_tile(p);
     a.total = (uint32_t)((int64_t)p.batch * p.dim * a.tiles_per_row);
     a.seqlen = p.seqlen; a.batch = p.batch; a.dim = p.dim;

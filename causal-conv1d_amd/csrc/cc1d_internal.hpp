@@ -65,7 +65,7 @@ struct Knob {
 };
 struct Tunables {
     Knob fwd_cl_rows, fwd_cl_half_vec, fwd_cl_chunk_runs, bwd_cl_rows, bwd_cl_chunk_runs, bwd_cl_lane_bytes,
-        fwd_cf_vecs, bwd_cf_parts, launch_limit_shift;
+        fwd_cf_vecs, bwd_cf_parts, bwd_cf_direct, launch_limit_shift;
 };
 Tunables &tunables();
 
@@ -111,10 +111,12 @@ size_t bwd_channelfirst_workspace_bytes(const cc1d_bwd_params &p);
 bool bwd_channellast_fits(const cc1d_bwd_params &p);
 bool bwd_channelfirst_fits(const cc1d_bwd_params &p);
 // Channel-first rows of more than 64 vectors: the tile kernel (cc1d_bwd_channelfirst_tile.hip);
-// its workspace is `parts` planes of (width + 1) x dim floats.
+// its workspace is `parts` planes of (width + 1) x dim floats.  `direct`: the kernel writes dweight and
+// dbias itself, there is no second stage.
 bool bwd_channelfirst_tile_applies(const cc1d_bwd_params &p);
 bool bwd_channelfirst_tile_fits(const cc1d_bwd_params &p);
 int bwd_channelfirst_tile_parts(const cc1d_bwd_params &p);
+bool bwd_channelfirst_tile_direct(const cc1d_bwd_params &p);
 int launch_bwd_channelfirst_tile(const cc1d_bwd_params &p, float *ws, hipStream_t stream);
 int launch_bwd_channellast(const cc1d_bwd_params &p, void *ws, hipStream_t stream);
 int launch_bwd_channelfirst(const cc1d_bwd_params &p, void *ws, hipStream_t stream);

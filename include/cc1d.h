@@ -282,6 +282,8 @@ int cc1d_hip_runtime_path(char *path, size_t size);
  *                   (0: 8 where the rows of dx do not start on 64-byte boundaries, else 4)
  *   "fwd_cf_vecs"   16-byte vectors per wave segment in the channel-first forward
  *   "bwd_cf_parts"  partitions of (batch x seqlen) per channel in the channel-first backward
+ *   "bwd_cf_direct" < 0: the channel-first backward never adds up a channel's partial sums in its own
+ *                   workgroup, also where that saves the second launch
  *   "launch_limit_shift" n: one launch holds at most 2^(31-n) threads instead of 2^31 (n <= 24), so
  *                   that small tensors exercise the batch slicing below
  *

@@ -1,0 +1,86 @@
+"""dweight / dbias of the channel-first tile kernel at the edges of the rule that picks who adds up a
+channel's tiles: the kernel's own workgroup (at most 16 tiles and 64 KiB of LDS, and at most two
+batch entries, a channel's rows adjacent in memory, or 8192 wavefronts) or the second launch
+(`bwd_cf_direct` = -1 forces it).  dx and dinitial_states must not depend on it; dweight and dbias are the
+same fp32 terms added in another order.  Taps of every type, packed and strided."""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import causal_conv1d_oracle as orc
+import cabi
+from helpers import TOL_W, assert_close, gen, make_states
+
+pytestmark = pytest.mark.gpu
+
+BF16, FP16, FP32 = torch.bfloat16, torch.float16, torch.float32
+CASES = [   # batch, dim, seqlen, width, dtype, weight dtype, strided weight, (dim, batch, seqlen) in memory
+    (1, 24, 513, 4, BF16, FP32, False, False),         # one tile of one step and a tail
+    (2, 24, 2049, 4, FP16, FP16, False, False),        # two tiles, the second a tail only
+    (2, 16, 12000, 3, BF16, BF16, True, False),        # 12 tiles of four steps
+    (14, 16, 1537, 4, BF16, BF16, False, False),       # 14 tiles of four steps: 61 KiB of LDS
+    (15, 16, 1990, 4, BF16, FP32, False, False),       # 15 of them: one more than fit
+    (16, 16, 1001, 2, FP32, FP32, True, False),        # 16 tiles
+    (17, 16, 600, 4, BF16, FP16, False, False),        # 17
+    (8, 1024, 520, 4, BF16, FP32, False, False),       # 8192 wavefronts
+    (8, 1032, 520, 4, BF16, FP32, False, False),       # 8256
+    (8, 1032, 520, 4, BF16, FP32, False, True),        # a channel's rows adjacent: any number
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(v).replace("torch.", "") for v in c))
+def test_sums_do_not_depend_on_who_adds_them(gpu_device, cc1d_lib, case):
+    lib, dev = cabi.declare(cc1d_lib), gpu_device
+    B, D, L, W, dtype, wtype, strided, batch_inner = case
+    g = gen(B * 1000 + L)
+
+    def tensor():
+        t = torch.randn(D, B, L, generator=g).transpose(0, 1) if batch_inner else torch.randn(B, D, L, generator=g)
+        return t.to(dtype)
+
+    x, dout = tensor(), tensor()
+    w = (torch.rand(D, 2 * W if strided else W, generator=g) - 0.5).to(wtype)
+    w = w[:, ::2] if strided else w
+    b = (torch.rand(D, generator=g) - 0.5).to(wtype)
+    init, dfin = make_states(B, D, W - 1, dtype, g), make_states(B, D, W - 1, dtype, g)
+    xd, dd, bd, initd, dfind = x.to(dev), dout.to(dev), b.to(dev), init.to(dev), dfin.to(dev)
+    wd = torch.empty(D, 2 * W, dtype=wtype, device=dev)[:, ::2] if strided else torch.empty(D, W, dtype=wtype, device=dev)
+    wd.copy_(w)
+
+    def run(knob):
+        dx = torch.empty_like(xd)
+        dinit = torch.empty(B, W - 1, D, device=dev, dtype=dtype).transpose(1, 2)
+        dw, db = torch.full((D, W), float("nan"), device=dev), torch.full((D,), float("nan"), device=dev)
+        got = []
+        for overwrite in (1, 0):                        # stored, then the same once more on top
+            p = cabi.bwd_params(xd, wd, bd, dd, dx, dw, db, True, initial_states=initd, dfinal_states=dfind,
+                                dinitial_states=dinit)
+            p.overwrite_dweight = overwrite
+            assert lib.cc1d_set_tunable(b"bwd_cf_direct", knob) == 0
+            try:
+                need = ctypes.c_size_t()
+                assert lib.cc1d_bwd_workspace_bytes(ctypes.byref(p), ctypes.byref(need)) == 0
+                ws = torch.empty(max(16, need.value), dtype=torch.uint8, device=dev)
+                stream = torch.cuda.current_stream().cuda_stream
+                assert lib.cc1d_bwd(ctypes.byref(p), ws.data_ptr(), need.value, stream) == 0
+                torch.cuda.synchronize()
+            finally:
+                lib.cc1d_set_tunable(b"bwd_cf_direct", 0)
+            got += [dw.clone(), db.clone()]
+        return [dx, dinit] + got
+
+    own, second = run(0), run(-1)
+    assert torch.equal(own[0], second[0]) and torch.equal(own[1], second[1])
+    assert torch.equal(own[4], 2 * own[2]) and torch.equal(own[5], 2 * own[3])
+    # At most 32 + 6 + 17 additions in a row per sum, of terms of at most 1.1 |dout| |x|: the two
+    # orders differ by no more than twice 55 roundings of the sum of the terms' magnitudes.
+    terms = 1.1 * dout.float().abs().sum((0, 2)) * x.float().abs().amax((0, 2)).clamp(min=1.0)
+    bound = (2 * 55 * 2.0 ** -24 * terms).to(dev)
+    assert bool(((own[2] - second[2]).abs() <= bound[:, None]).all())
+    assert bool(((own[3] - second[3]).abs() <= bound).all())
+    rdx, rdw, rdb, rdi = orc.bwd(x, w.float().contiguous(), b.float(), dout, initial_states=init, dfinal_states=dfin, activation="silu")
+    assert_close(own[0], rdx, dtype, "dx")
+    assert_close(own[1], rdi, dtype, "dinitial_states")
+    assert_close(own[2], rdw, what="dweight", tol=TOL_W)
+    assert_close(own[3], rdb, what="dbias", tol=TOL_W)
