@@ -98,7 +98,7 @@ __device__ __forceinline__ float wave_total_in_lane63(float v) {
 // DIRECT: a workgroup is one channel and its wavefronts are the channel's tiles, so that it can add up
 // their sums itself and store dweight / dbias: one launch instead of two, and no workspace
 // traffic.  Otherwise the wavefronts are numbered along the rows, four to a workgroup, and leave their
-// sums to the second stage.  See tile_sums_directly for the line between the two.
+// sums to the second stage.  See bwd_channelfirst_tile_direct for the line between the two.
 // Registers: 64 at most (16-bit data), so that eight wavefronts share a SIMD; wave-uniform values
 // (taps, the odd last element, dfinal_states) live in scalar registers for that.  The launch is bound
 // by memory and by the vector ALUs about equally, and what counts is how well the two overlap:
