@@ -136,7 +136,7 @@ def build_binding(force=False, out_dir=None):
             src, "-o", out]
     for lp in ce.library_paths():
         cmd += ["-L" + lp, "-Wl,-rpath," + lp]
-    cmd += ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python",
+    cmd += ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python",
             "-L" + HERE, "-l:" + LIB_NAME, "-Wl,-rpath,$ORIGIN"]
     _run(cmd)
     return out

@@ -10,6 +10,12 @@
 // allocates is the backward workspace, through the caching allocator.
 #include <torch/extension.h>
 #include <torch/library.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/core/dispatch/Dispatcher.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
@@ -380,13 +386,21 @@ void fwd_op(const at::Tensor &x, const at::Tensor &weight, const std::optional<a
     causal_conv1d_fwd(x, weight, bias, seq_idx, initial_states, out, fin, silu_activation);
 }
 
+// An uninitialised tensor laid out like x, as at::empty_like gives it.  Dense GPU tensors (any order of
+// strides) skip the two dispatcher hops of empty_like + empty_strided, 0.5 us a call.
+at::Tensor uninitialised_like(const at::Tensor &x) {
+    if (x.is_cuda() && x.is_non_overlapping_and_dense())
+        return at::Tensor(at::detail::empty_strided_cuda(x.sizes(), x.strides(), x.scalar_type(), x.device()));
+    return at::empty_like(x);
+}
+
 // The forward with its result allocated here, in x's layout: one dispatcher hop and no
 // empty_like in Python (about a microsecond of host time, which is what a short prefill is
 // bound by).  Not an op of the reference.
 at::Tensor fwd_out_op(const at::Tensor &x, const at::Tensor &weight, const std::optional<at::Tensor> &bias,
                       const std::optional<at::Tensor> &seq_idx, const std::optional<at::Tensor> &initial_states,
                       const std::optional<at::Tensor> &final_states_out, bool silu_activation) {
-    at::Tensor out = at::empty_like(x);
+    at::Tensor out = uninitialised_like(x);
     std::optional<at::Tensor> fin = final_states_out;
     causal_conv1d_fwd(x, weight, bias, seq_idx, initial_states, out, fin, silu_activation);
     return out;
@@ -437,7 +451,7 @@ at::Tensor update_out_op(const at::Tensor &x, at::Tensor &conv_state, const at::
                          const std::optional<at::Tensor> &cache_seqlens,
                          const std::optional<at::Tensor> &conv_state_indices) {
     TORCH_CHECK(x.dim() == 2 || x.dim() == 3, "x must be (batch, dim) or (batch, dim, seqlen)");
-    at::Tensor out = at::empty_like(x);
+    at::Tensor out = uninitialised_like(x);
     causal_conv1d_update(x, conv_state, weight, bias, out, silu_activation, cache_seqlens, conv_state_indices);
     return out;
 }
@@ -457,6 +471,144 @@ void bwd_meta(const at::Tensor &, const at::Tensor &, const std::optional<at::Te
 void update_meta(const at::Tensor &, at::Tensor &, const at::Tensor &, const std::optional<at::Tensor> &,
                  at::Tensor &, bool, const std::optional<at::Tensor> &, const std::optional<at::Tensor> &) {}
 
+// ---- direct calls from Python ---------------------------------------------------------
+// The package's functions reach the dispatcher through these instead of through torch.ops: the same
+// ops, called with plain C++ arguments.  What is left out is the generic parsing of Python arguments
+// against the op's schema into a stack of boxed values and back, about 2 us of the 5 us of host time
+// that a decode step took, which is what bounds a decode step of up to about 100 requests.  Everything behind
+// the dispatcher (autograd's handling, fake tensors, dispatch modes, profiling) sees the same call.
+// Each returns NotImplemented, having done nothing, for what the generic path in Python has to
+// handle: tensor subclasses, torch-function modes, tracing, arguments of other types or that still need a copy.
+
+bool plain(PyObject *o) { return THPVariable_CheckExact(o); }
+bool plain_or_none(PyObject *o) { return o == Py_None || plain(o); }
+std::optional<at::Tensor> optional_tensor(PyObject *o) {
+    return o == Py_None ? std::optional<at::Tensor>() : std::optional<at::Tensor>(THPVariable_Unpack(o));
+}
+bool generic_path_needed() {
+    return at::impl::torch_function_mode_enabled() || torch::jit::tracer::isTracing();
+}
+// Unit stride along seqlen or along dim.
+bool kernel_layout(const at::Tensor &t) { return t.dim() == 3 && (t.stride(1) == 1 || t.stride(2) == 1); }
+bool contiguous_or_none(const std::optional<at::Tensor> &t) { return !t.has_value() || t->is_contiguous(); }
+
+// A (batch, dim, width - 1) tensor with unit stride along dim.
+at::Tensor states_like(const at::Tensor &x, int64_t width) {
+    return at::empty({x.size(0), width - 1, x.size(1)}, x.options()).transpose(1, 2);
+}
+
+template <typename F>
+auto typed_op(const char *name) {
+    return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<F>();
+}
+
+#define NOT_IMPLEMENTED() do { Py_INCREF(Py_NotImplemented); return Py_NotImplemented; } while (0)
+
+// (x, conv_state, weight, bias, silu, cache_seqlens, conv_state_indices) -> out
+PyObject *update_call(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 7 || !plain(a[0]) || !plain(a[1]) || !plain(a[2]) || !plain_or_none(a[3]) || !PyBool_Check(a[4]) ||
+        !plain_or_none(a[5]) || !plain_or_none(a[6]) || generic_path_needed())
+        NOT_IMPLEMENTED();
+    static const auto op = typed_op<decltype(update_out_op)>("DaoAILab::_causal_conv1d_update_out_cpp");
+    at::Tensor state = THPVariable_Unpack(a[1]);
+    const at::Tensor x = THPVariable_Unpack(a[0]), weight = THPVariable_Unpack(a[2]);
+    const auto bias = optional_tensor(a[3]), lengths = optional_tensor(a[5]), indices = optional_tensor(a[6]);
+    const bool silu = a[4] == Py_True;
+    at::Tensor out;
+    {
+        pybind11::gil_scoped_release no_gil;
+        out = op.call(x, state, weight, bias, silu, lengths, indices);
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// (x, weight, bias, seq_idx, initial_states, return_final_states, final_states_out, silu)
+// -> out or (out, final_states).  Tensors that still need a copy into a layout of the kernels, and
+// combinations that the Python layer refuses, are left to it.
+PyObject *forward_call(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 8 || !plain(a[0]) || !plain(a[1]) || !plain_or_none(a[2]) || !plain_or_none(a[3]) || !plain_or_none(a[4]) ||
+        !PyBool_Check(a[5]) || !plain_or_none(a[6]) || !PyBool_Check(a[7]) || generic_path_needed())
+        NOT_IMPLEMENTED();
+    static const auto op = typed_op<decltype(fwd_out_op)>("DaoAILab::_causal_conv1d_fwd_out_cpp");
+    const at::Tensor x = THPVariable_Unpack(a[0]), weight = THPVariable_Unpack(a[1]);
+    const auto bias = optional_tensor(a[2]), seq_idx = optional_tensor(a[3]), init = optional_tensor(a[4]);
+    const bool return_final = a[5] == Py_True, silu = a[7] == Py_True;
+    std::optional<at::Tensor> fin = return_final ? optional_tensor(a[6]) : std::nullopt;
+    if (!kernel_layout(x) || weight.dim() != 2 || !contiguous_or_none(bias) || !contiguous_or_none(seq_idx) ||
+        (init.has_value() && !kernel_layout(*init)) || (fin.has_value() && !kernel_layout(*fin)) ||
+        (seq_idx.has_value() && (init.has_value() || return_final)))
+        NOT_IMPLEMENTED();
+    at::Tensor out;
+    {
+        pybind11::gil_scoped_release no_gil;
+        if (return_final && !fin.has_value()) fin = states_like(x, weight.size(1));
+        out = op.call(x, weight, bias, seq_idx, init, fin, silu);
+    }
+    if (!return_final) return THPVariable_Wrap(std::move(out));
+    PyObject *pair = PyTuple_New(2);
+    if (pair == nullptr) throw python_error();
+    PyTuple_SET_ITEM(pair, 0, THPVariable_Wrap(std::move(out)));
+    if (a[6] != Py_None) {                              // the caller's own object
+        Py_INCREF(a[6]);
+        PyTuple_SET_ITEM(pair, 1, a[6]);
+    } else {
+        PyTuple_SET_ITEM(pair, 1, THPVariable_Wrap(std::move(*fin)));
+    }
+    return pair;
+    END_HANDLE_TH_ERRORS
+}
+
+// (x, weight, bias, dout, seq_idx, initial_states, dfinal_states, return_dinitial_states, silu)
+// -> (dx, dweight, dbias, dinitial_states): every output allocated here, dweight and dbias summed in
+// one fp32 buffer and converted to the parameters' type.
+PyObject *backward_call(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 9 || !plain(a[0]) || !plain(a[1]) || !plain_or_none(a[2]) || !plain(a[3]) || !plain_or_none(a[4]) ||
+        !plain_or_none(a[5]) || !plain_or_none(a[6]) || !PyBool_Check(a[7]) || !PyBool_Check(a[8]) || generic_path_needed())
+        NOT_IMPLEMENTED();
+    static const auto op = typed_op<decltype(bwd_overwrite_op)>("DaoAILab::_causal_conv1d_bwd_overwrite_cpp");
+    const at::Tensor x = THPVariable_Unpack(a[0]), weight = THPVariable_Unpack(a[1]), dout = THPVariable_Unpack(a[3]);
+    const auto bias = optional_tensor(a[2]), seq_idx = optional_tensor(a[4]), init = optional_tensor(a[5]), dfinal = optional_tensor(a[6]);
+    if (x.dim() != 3 || weight.dim() != 2 || !kernel_layout(dout)) NOT_IMPLEMENTED();
+    const bool return_dinit = a[7] == Py_True, silu = a[8] == Py_True;
+    at::Tensor dx, dweight;
+    std::optional<at::Tensor> dbias, dinit;
+    {
+        pybind11::gil_scoped_release no_gil;
+        const int64_t dim = weight.size(0), width = weight.size(1);
+        dx = at::empty_like(x);
+        const at::Tensor sums = at::empty({dim * (width + (bias.has_value() ? 1 : 0))}, x.options().dtype(at::kFloat));
+        dweight = sums.narrow(0, 0, dim * width).view({dim, width});
+        if (bias.has_value()) dbias = sums.narrow(0, dim * width, dim);
+        if (return_dinit) dinit = states_like(x, width);
+        op.call(x, weight, bias, dout, seq_idx, init, dfinal, dx, dweight, dbias, dinit, silu);
+        dweight = dweight.type_as(weight);
+        if (bias.has_value()) dbias = dbias->type_as(*bias);
+    }
+    PyObject *all = PyTuple_New(4);
+    if (all == nullptr) throw python_error();
+    PyTuple_SET_ITEM(all, 0, THPVariable_Wrap(std::move(dx)));
+    PyTuple_SET_ITEM(all, 1, THPVariable_Wrap(std::move(dweight)));
+    for (int i = 2; i < 4; ++i) {
+        std::optional<at::Tensor> &t = i == 2 ? dbias : dinit;
+        PyObject *o = Py_None;
+        if (t.has_value()) o = THPVariable_Wrap(std::move(*t));
+        else Py_INCREF(o);
+        PyTuple_SET_ITEM(all, i, o);
+    }
+    return all;
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef direct_calls[] = {
+    {"_update_call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&update_call)), METH_FASTCALL, nullptr},
+    {"_forward_call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&forward_call)), METH_FASTCALL, nullptr},
+    {"_backward_call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&backward_call)), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -466,6 +618,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("causal_conv1d_varlen_states", &causal_conv1d_varlen_states, "Varlen final-state gather");
     m.def("causal_conv1d_fwd_varlen_states", &causal_conv1d_fwd_varlen_states,
           "Causal conv1d forward and varlen final-state gather in one call");
+    if (PyModule_AddFunctions(m.ptr(), direct_calls) != 0) throw pybind11::error_already_set();
 }
 
 TORCH_LIBRARY_FRAGMENT(DaoAILab, m) {
