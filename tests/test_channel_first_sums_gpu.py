@@ -1,7 +1,7 @@
-"""dweight / dbias of the channel-first tile kernel at the edges of the rule that picks who adds up a
+"""dweight / dbias of the channel-first kernels at the edges of the rule that picks who adds up a
 channel's tiles: the kernel's own workgroup (at most 16 tiles and 64 KiB of LDS, and at most two
-batch entries, a channel's rows adjacent in memory, or 8192 wavefronts) or the second launch
-(`bwd_cf_direct` = -1 forces it).  dx and dinitial_states must not depend on it; dweight and dbias are the
+batch entries, a channel's rows adjacent in memory, or 8192 wavefronts; rows of at most 64 vectors: 2 to 16
+parts) or the second launch (`bwd_cf_direct` = -1 forces it).  dx and dinitial_states must not depend on it; dweight and dbias are the
 same fp32 terms added in another order.  Taps of every type, packed and strided."""
 import ctypes
 
@@ -26,6 +26,13 @@ CASES = [   # batch, dim, seqlen, width, dtype, weight dtype, strided weight, (d
     (8, 1024, 520, 4, BF16, FP32, False, False),       # 8192 wavefronts
     (8, 1032, 520, 4, BF16, FP32, False, False),       # 8256
     (8, 1032, 520, 4, BF16, FP32, False, True),        # a channel's rows adjacent: any number
+    (1, 24, 512, 4, BF16, FP32, False, False),         # short rows: one part
+    (2, 24, 512, 4, BF16, BF16, False, False),         # two parts
+    (16, 24, 505, 3, FP16, FP32, True, False),         # 16, rows off the vector grid
+    (17, 24, 256, 4, FP32, FP32, False, False),        # 17
+    (64, 24, 60, 2, BF16, FP32, False, False),         # eight rows to a wavefront, eight parts
+    (100, 24, 1, 4, FP32, FP32, False, False),         # rows of one element, two parts
+    (5, 1500, 100, 4, FP16, FP16, False, True),        # parts of several wavefronts' rows
 ]
 
 
