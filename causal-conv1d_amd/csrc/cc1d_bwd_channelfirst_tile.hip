@@ -358,7 +358,9 @@ bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
     dB = wave_total_in_lane63(dB);
     if constexpr (DIRECT) {
         // The channel's tiles are this workgroup's wavefronts: their sums are added in order and stored.
-        const int waves = (int)(blockDim.x / kWave);
+        // (not blockDim: a kernel that asks for its launch shape takes 256 bytes of hidden arguments, and
+        // every byte of a launch's arguments costs about 3 ns of host time)
+        const int waves = a.batch * (int)a.tiles_per_row;
         float *sums = reinterpret_cast<float *>(lds + waves * XV);
         if (lane == kWave - 1) {
 #pragma unroll
