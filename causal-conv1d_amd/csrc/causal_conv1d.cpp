@@ -387,7 +387,7 @@ void fwd_op(const at::Tensor &x, const at::Tensor &weight, const std::optional<a
 }
 
 // An uninitialised tensor laid out like x, as at::empty_like gives it.  Dense GPU tensors (any order of
-// strides) skip the two dispatcher hops of empty_like + empty_strided, 0.5 us a call.
+// strides) skip the two dispatcher hops of empty_like and empty_strided.
 at::Tensor uninitialised_like(const at::Tensor &x) {
     if (x.is_cuda() && x.is_non_overlapping_and_dense())
         return at::Tensor(at::detail::empty_strided_cuda(x.sizes(), x.strides(), x.scalar_type(), x.device()));
@@ -474,9 +474,9 @@ void update_meta(const at::Tensor &, at::Tensor &, const at::Tensor &, const std
 // ---- direct calls from Python ---------------------------------------------------------
 // The package's functions reach the dispatcher through these instead of through torch.ops: the same
 // ops, called with plain C++ arguments.  What is left out is the generic parsing of Python arguments
-// against the op's schema into a stack of boxed values and back, about 2 us of the 5 us of host time
-// that a decode step took, which is what bounds a decode step of up to about 100 requests.  Everything behind
-// the dispatcher (autograd's handling, fake tensors, dispatch modes, profiling) sees the same call.
+// against the op's schema into a stack of boxed values and back: 1.1 instead of 2.0 us of host time for
+// a decode call without its launch.  32 layers of one request, which the host bounds: 178 -> 149 us,
+// uninitialised_like included.  Everything behind the dispatcher (autograd's handling, fake tensors, dispatch modes, profiling) sees the same call.
 // Each returns NotImplemented, having done nothing, for what the generic path in Python has to
 // handle: tensor subclasses, torch-function modes, tracing, arguments of other types or that still need a copy.
 

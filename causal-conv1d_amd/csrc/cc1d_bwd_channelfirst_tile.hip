@@ -13,8 +13,8 @@
 // (buffer_load_dwordx4 ... lds), where a lane finds its neighbours' elements, together with the
 // vector in front of the tile (the x halo) and the vectors behind it (the W-1 positions whose g
 // the tile's last lane needs); dout, which only the lane that owns it reads, goes to registers
-// (four per step: with LDS for one tensor instead of two, seven wavefronts share a SIMD instead
-// of four: 1-3 % at most shapes, (2, 2048, 16384) bf16 71.1 -> 69.2 us).  The launch is thousands of wavefronts
+// (four per step: with LDS for one tensor instead of two, LDS no longer holds a SIMD to four wavefronts,
+// which then was worth 1-3 % at most shapes, (2, 2048, 16384) bf16 71.1 -> 69.2 us).  The launch is thousands of wavefronts
 // that live for one memory round trip and a few hundred instructions each and sweep through
 // memory as one compact front in the order of the rows -- where one long-lived wavefront per
 // channel walks 4096 far-apart streams at once, which is what bounds that design at the
