@@ -82,37 +82,16 @@ namespace {
 
 constexpr int kXcds = 8;
 
-// The lane's columns of the rows of one run; row i is `stride` bytes behind row i - 1, row 0 the run's
-// first.  Two forms of the same access:
-//  * PointerRows: a 64-bit address per lane.
-//  * ResourceRows: the row is a scalar offset into a buffer resource and the lane one 32-bit offset that
-//    never changes.  No register pair and no vector instruction goes into addresses, but the offsets
-//    cost scalar registers and instructions in front of the walk.
+// The lane's columns of the rows of one run through a buffer resource: the row is a scalar offset and
+// the lane one 32-bit offset that never changes.  Row i is `stride` bytes behind row i - 1, row 0 the
+// run's first.  Against a 64-bit address per lane, no register pair and no vector instruction goes into
+// addresses, but the offsets cost scalar registers and instructions in front of the walk.
 // fp16 with seq_idx and width 4 takes resources: with pointers its walk does not fit the 128 registers
 // that four workgroups per CU leave it (13 spilled): (8, 5376, 2048) 109.1 -> 93.7 us, (16, 2048, 2048)
 // 93.9 -> 74.6.  Everything else fits either way and keeps pointers: (8, 5376, 2048) bf16 93.7 / 94.2 us
-// (pointers / resources), (4, 4096, 4096) 73.1 / 73.7, (1, 5376, 512) 10.9 / 11.4.
-template <typename raw_t, int HALO>
-struct PointerRows {
-    char *run;
-    uint32_t stride;
-    __device__ __forceinline__ PointerRows(const void *row0, int lane_off, uint32_t bytes)
-        : run(const_cast<char *>(static_cast<const char *>(row0)) + lane_off), stride(bytes) {}
-    __device__ __forceinline__ raw_t halo(int rows_in_front) const {
-        return *reinterpret_cast<const raw_t *>(run - (int64_t)rows_in_front * stride);
-    }
-    template <bool STREAM>
-    __device__ __forceinline__ raw_t load(int i) const {
-        const raw_t *src = reinterpret_cast<const raw_t *>(run + (uint32_t)i * stride);
-        return STREAM ? __builtin_nontemporal_load(src) : *src;
-    }
-    template <bool STREAM>
-    __device__ __forceinline__ void store(int i, const raw_t &v) const {
-        raw_t *dst = reinterpret_cast<raw_t *>(run + (uint32_t)i * stride);
-        if (STREAM) __builtin_nontemporal_store(v, dst);
-        else *dst = v;
-    }
-};
+// (pointers / resources), (4, 4096, 4096) 73.1 / 73.7, (1, 5376, 512) 10.9 / 11.4.  The pointers stay
+// written out where they are used: wrapped in a type like this one they compile to other code in every
+// kernel, with seq_idx up to 5 % slower ((1, 8192, 1500) bf16 22.9 -> 23.6 us, (1, 5376, 64) fp32 9.5 -> 10.0).
 template <typename raw_t, int HALO>
 struct ResourceRows {
     static_assert(sizeof(raw_t) == 4, "4-byte lanes");
@@ -137,6 +116,10 @@ struct ResourceRows {
     __device__ __forceinline__ void store(int i, const raw_t &v) const {
         __builtin_amdgcn_raw_buffer_store_b32(v[0], rsrc, lane_off, (HALO + i) * stride, STREAM ? 2 : 0);
     }
+};
+
+struct NoRows {
+    __device__ __forceinline__ NoRows(const void *, int, uint32_t) {}
 };
 
 constexpr int kRunsPerBlock = kBlock / kWave;   // the wavefronts of a workgroup take consecutive runs
@@ -169,18 +152,23 @@ bwd_channellast_run(const cc1d_bwd_params &p, const BwdClGeom &g, const int32_t 
     if (WM != 0) taps.request(p.weight, p.bias, c0);
     else any_taps.request(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, c0);
 
-    // Rows of this run; offsets inside a run fit 31 bits (checked by the launcher).  Row i of the walk
-    // stores dx row i-(W-1): dx is moved back once instead.
+    // Row pointers of this run; offsets inside a run fit 31 bits (checked by the launcher).
+    const char *xrun = reinterpret_cast<const char *>(reinterpret_cast<const T_ *>(p.x) + (int64_t)b * p.x_stride_b + c0 + (int64_t)t0 * p.x_stride_l);
+    const char *drun = reinterpret_cast<const char *>(reinterpret_cast<const T_ *>(p.dout) + (int64_t)b * p.dout_stride_b + c0 + (int64_t)t0 * p.dout_stride_l);
+    // Row i of the walk stores dx row i-(W-1): the pointer is moved back once instead.
+    char *dxrun = reinterpret_cast<char *>(reinterpret_cast<T_ *>(p.dx) + (int64_t)b * p.dx_stride_b + c0) +
+                  ((int64_t)t0 - (W - 1)) * p.dx_stride_l * (int64_t)sizeof(T_);
+    const uint32_t xs = (uint32_t)p.x_stride_l * (uint32_t)sizeof(T_);
+    const uint32_t ds = (uint32_t)p.dout_stride_l * (uint32_t)sizeof(T_);
+    const uint32_t dxs = (uint32_t)p.dx_stride_l * (uint32_t)sizeof(T_);
+    // The same rows as resources.
     constexpr bool RESOURCES = DT == CC1D_F16 && CH == 2 && HAS_SEQ && W == 4;
-    using InRows = std::conditional_t<RESOURCES, ResourceRows<raw_t, 2 * (W - 1)>, PointerRows<raw_t, 2 * (W - 1)>>;
-    using OutRows = std::conditional_t<RESOURCES, ResourceRows<raw_t, 0>, PointerRows<raw_t, 0>>;
+    using Rows = std::conditional_t<RESOURCES, ResourceRows<raw_t, 2 * (W - 1)>, NoRows>;
+    using OutRows = std::conditional_t<RESOURCES, ResourceRows<raw_t, 0>, NoRows>;
     const int lane_off = c0 * (int)sizeof(T_);
-    const InRows xrows(reinterpret_cast<const T_ *>(p.x) + (int64_t)b * p.x_stride_b + (int64_t)t0 * p.x_stride_l, lane_off,
-                       (uint32_t)p.x_stride_l * (uint32_t)sizeof(T_));
-    const InRows drows(reinterpret_cast<const T_ *>(p.dout) + (int64_t)b * p.dout_stride_b + (int64_t)t0 * p.dout_stride_l, lane_off,
-                       (uint32_t)p.dout_stride_l * (uint32_t)sizeof(T_));
-    const OutRows dxrows(reinterpret_cast<T_ *>(p.dx) + (int64_t)b * p.dx_stride_b + ((int64_t)t0 - (W - 1)) * p.dx_stride_l, lane_off,
-                         (uint32_t)p.dx_stride_l * (uint32_t)sizeof(T_));
+    const Rows xrows(reinterpret_cast<const T_ *>(p.x) + (int64_t)b * p.x_stride_b + (int64_t)t0 * p.x_stride_l, lane_off, xs);
+    const Rows drows(reinterpret_cast<const T_ *>(p.dout) + (int64_t)b * p.dout_stride_b + (int64_t)t0 * p.dout_stride_l, lane_off, ds);
+    const OutRows dxrows(reinterpret_cast<T_ *>(p.dx) + (int64_t)b * p.dx_stride_b + ((int64_t)t0 - (W - 1)) * p.dx_stride_l, lane_off, dxs);
     // seq_idx is a kernel argument of its own, marked as not aliasing anything the kernel
     // writes: its loads, at wave-uniform addresses, go through the scalar cache.
     const int32_t *seq = HAS_SEQ ? seq_idx + (int64_t)b * L + t0 : nullptr;
@@ -239,7 +227,8 @@ bwd_channellast_run(const cc1d_bwd_params &p, const BwdClGeom &g, const int32_t 
         const int t = t0 - 2 * (W - 1) + q;
         xh_raw[q] = P::zero();
         if (t >= 0) {
-            xh_raw[q] = xrows.halo(2 * (W - 1) - q);
+            if constexpr (RESOURCES) xh_raw[q] = xrows.halo(2 * (W - 1) - q);
+            else xh_raw[q] = *reinterpret_cast<const raw_t *>(xrun - (int64_t)(2 * (W - 1) - q) * xs);
         } else if (p.initial_states != nullptr && t >= -(W - 1)) {
             xh_raw[q] = load_state_row<DT, CH>(p.initial_states, p.init_stride_b, p.init_stride_c,
                                                p.init_stride_l, b, c0, t + (W - 1));
@@ -250,7 +239,10 @@ bwd_channellast_run(const cc1d_bwd_params &p, const BwdClGeom &g, const int32_t 
     for (int k = 0; k < W - 1; ++k) {
         const int t = t0 - (W - 1) + k;
         dh_raw[k] = P::zero();
-        if (t >= 0) dh_raw[k] = drows.halo(W - 1 - k);
+        if (t >= 0) {
+            if constexpr (RESOURCES) dh_raw[k] = drows.halo(W - 1 - k);
+            else dh_raw[k] = *reinterpret_cast<const raw_t *>(drun - (int64_t)(W - 1 - k) * ds);
+        }
     }
     auto fill_windows = [&]() __attribute__((always_inline)) {
         if (WM != 0) taps.finish(p.bias != nullptr, wv, bv);
@@ -327,8 +319,15 @@ bwd_channellast_run(const cc1d_bwd_params &p, const BwdClGeom &g, const int32_t 
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int i = (!decltype(checked)::value || (i0 + u) < last) ? (i0 + u) : last;
-            rx[u] = xrows.template load<decltype(stream)::value>(i);
-            rd[u] = drows.template load<decltype(stream)::value>(i);
+            if constexpr (RESOURCES) {
+                rx[u] = xrows.template load<decltype(stream)::value>(i);
+                rd[u] = drows.template load<decltype(stream)::value>(i);
+            } else {
+                const raw_t *sx = reinterpret_cast<const raw_t *>(xrun + (uint32_t)i * xs);
+                const raw_t *sd = reinterpret_cast<const raw_t *>(drun + (uint32_t)i * ds);
+                rx[u] = decltype(stream)::value ? __builtin_nontemporal_load(sx) : *sx;
+                rd[u] = decltype(stream)::value ? __builtin_nontemporal_load(sd) : *sd;
+            }
             sq[u] = HAS_SEQ ? seq[i] : 0;
         }
     };
@@ -355,12 +354,15 @@ bwd_channellast_run(const cc1d_bwd_params &p, const BwdClGeom &g, const int32_t 
             }
             dx_row(masked, gw, sqw, gv, cur, dxv);
             if (!decltype(checked)::value) {
-                dxrows.template store<CC1D_BWD_CL_STREAM_STORES != 0>(i0 + u, P::pack(dxv));
+                if constexpr (RESOURCES) dxrows.template store<CC1D_BWD_CL_STREAM_STORES != 0>(i0 + u, P::pack(dxv));
+                else if (CC1D_BWD_CL_STREAM_STORES) __builtin_nontemporal_store(P::pack(dxv), reinterpret_cast<raw_t *>(dxrun + (uint32_t)(i0 + u) * dxs));
+                else *reinterpret_cast<raw_t *>(dxrun + (uint32_t)(i0 + u) * dxs) = P::pack(dxv);
             } else {
                 // Row t < L completes position pp = t-(W-1) < L-(W-1): no dfinal term yet.
                 const int pp = t0 + i0 + u - (W - 1);
                 if (pp >= 0) {
-                    dxrows.template store<false>(i0 + u, P::pack(dxv));
+                    if constexpr (RESOURCES) dxrows.template store<false>(i0 + u, P::pack(dxv));
+                    else *reinterpret_cast<raw_t *>(dxrun + (int64_t)(i0 + u) * dxs) = P::pack(dxv);
                 } else if (p.dinitial_states != nullptr) {
                     store_state_row<DT, CH>(p.dinitial_states, p.dinit_stride_b, p.dinit_stride_c,
                                             p.dinit_stride_l, b, c0, pp + (W - 1), P::pack(dxv));
