@@ -86,12 +86,12 @@ constexpr int kXcds = 8;
 // the lane one 32-bit offset that never changes.  Row i is `stride` bytes behind row i - 1, row 0 the
 // run's first.  Against a 64-bit address per lane, no register pair and no vector instruction goes into
 // addresses, but the offsets cost scalar registers and instructions in front of the walk.
-// fp16 with seq_idx and width 4 takes resources: with pointers its walk does not fit the 128 registers
-// that four workgroups per CU leave it (13 spilled): (8, 5376, 2048) 109.1 -> 93.7 us, (16, 2048, 2048)
-// 93.9 -> 74.6.  Everything else fits either way and keeps pointers: (8, 5376, 2048) bf16 93.7 / 94.2 us
-// (pointers / resources), (4, 4096, 4096) 73.1 / 73.7, (1, 5376, 512) 10.9 / 11.4.  The pointers stay
-// written out where they are used: wrapped in a type like this one they compile to other code in every
-// kernel, with seq_idx up to 5 % slower ((1, 8192, 1500) bf16 22.9 -> 23.6 us, (1, 5376, 64) fp32 9.5 -> 10.0).
+// The kernel's RESOURCES form of fp16 with seq_idx, width 4 and SiLU takes them (see takes_resources):
+// with pointers that walk does not fit the 128 registers that four workgroups per CU leave it (13 spilled).
+// Everything else fits either way and keeps pointers: (8, 5376, 2048) bf16 93.7 / 94.2 us (pointers /
+// resources), (4, 4096, 4096) 73.1 / 73.7, (1, 5376, 512) 10.9 / 11.4.  The pointers stay written out where
+// they are used: wrapped in a type like this one they compile to other code in every kernel, with seq_idx
+// up to 5 % slower ((1, 8192, 1500) bf16 22.9 -> 23.6 us, (1, 5376, 64) fp32 9.5 -> 10.0).
 template <typename raw_t, int HALO>
 struct ResourceRows {
     static_assert(sizeof(raw_t) == 4, "4-byte lanes");
@@ -126,7 +126,7 @@ constexpr int kRunsPerBlock = kBlock / kWave;   // the wavefronts of a workgroup
 
 // One wavefront's walk over run `run` of sequence b, columns col*CH .. col*CH+CH per lane: writes
 // dx (and dinitial_states) and returns the lane's dweight / dbias terms in dW / dB.
-template <int DT, int CH, int W, bool HAS_SEQ, bool SILU, int U, int WM>
+template <int DT, int CH, int W, bool HAS_SEQ, bool SILU, int U, int WM, bool RESOURCES>
 __device__ __forceinline__ void
 bwd_channellast_run(const cc1d_bwd_params &p, const BwdClGeom &g, const int32_t *__restrict__ seq_idx,
                     const int b, const int run, const uint32_t col, float (&dW)[CH][W], float (&dB)[CH]) {
@@ -162,7 +162,6 @@ bwd_channellast_run(const cc1d_bwd_params &p, const BwdClGeom &g, const int32_t 
     const uint32_t ds = (uint32_t)p.dout_stride_l * (uint32_t)sizeof(T_);
     const uint32_t dxs = (uint32_t)p.dx_stride_l * (uint32_t)sizeof(T_);
     // The same rows as resources.
-    constexpr bool RESOURCES = DT == CC1D_F16 && CH == 2 && HAS_SEQ && W == 4;
     using Rows = std::conditional_t<RESOURCES, ResourceRows<raw_t, 2 * (W - 1)>, NoRows>;
     using OutRows = std::conditional_t<RESOURCES, ResourceRows<raw_t, 0>, NoRows>;
     const int lane_off = c0 * (int)sizeof(T_);
@@ -466,8 +465,9 @@ bwd_channellast_run(const cc1d_bwd_params &p, const BwdClGeom &g, const int32_t 
 }
 
 // WM: how the taps are read.  1: packed (dim, W) fp32, 2: packed in x's own 16-bit type (both
-// through PackedTaps), 0: any layout and type (general loader).
-template <int DT, int CH, int W, bool HAS_SEQ, bool SILU, int U, int WM>
+// through PackedTaps), 0: any layout and type (general loader).  RESOURCES: rows through buffer
+// resources instead of pointers (see ResourceRows).
+template <int DT, int CH, int W, bool HAS_SEQ, bool SILU, int U, int WM, bool RESOURCES>
 __global__ void __launch_bounds__(kBlock, (CH * Elem<DT>::kBytes == 4 ? CC1D_BWD_CL_OCC : CC1D_BWD_CL_OCC8))
 bwd_channellast_kernel(const cc1d_bwd_params p, const BwdClGeom g, float *__restrict__ ws,
                        const int32_t *__restrict__ seq_idx) {
@@ -501,7 +501,7 @@ bwd_channellast_kernel(const cc1d_bwd_params p, const BwdClGeom g, float *__rest
     // Workgroups past the end of the grid's last XCD slice, runs past the end of the sequence
     // and lanes past the last column have nothing to walk; they still meet the barrier below.
     const bool active = block < g.total && run < g.n_runs && col < (uint32_t)g.n_colgroups;
-    if (active) bwd_channellast_run<DT, CH, W, HAS_SEQ, SILU, U, WM>(p, g, seq_idx, b, run, col, dW, dB);
+    if (active) bwd_channellast_run<DT, CH, W, HAS_SEQ, SILU, U, WM, RESOURCES>(p, g, seq_idx, b, run, col, dW, dB);
 
     // The workgroup's four partial sums are added in the order of the runs and stored once:
     // plane w of part (b, quad), channels c0 .. c0+CH.
@@ -532,14 +532,33 @@ bwd_channellast_kernel(const cc1d_bwd_params p, const BwdClGeom g, float *__rest
 }
 
 
+// Whether a launch of the one kernel that spills with pointers (fp16, seq_idx, width 4, SiLU, 4-byte lanes)
+// names its rows by resources: from more than one wavefront per SIMD on.  Up to there the spills cost
+// less than the instructions in front of the walk.  Pointers / resources, us, wavefronts in brackets:
+// (1, 1024, 2048) [512] 12.9 / 13.3, (1, 5376, 512) [672] 13.2 / 13.6, (2, 2048, 1001) [1024] 13.6 / 13.8,
+// (10, 1024, 512) [1280] 16.4 / 15.8, (1, 5376, 1024) [1344] 16.1 / 15.6, (8, 1024, 2048) 28.8 / 25.0,
+// (8, 5376, 2048) 110.4 / 94.4, (16, 2048, 2048) 90.2 / 76.4.  Without the activation nothing spills and resources
+// are slower: (1, 5376, 512) 11.5 / 12.1, (8, 5376, 2048) 92.2 / 94.2.
+inline bool takes_resources(const cc1d_bwd_params &p, const BwdClGeom &g) {
+    constexpr int64_t kSimds = 256 * 4;
+    return (int64_t)p.batch * g.n_runs * g.waves_per_row > kSimds;
+}
+
 template <int DT, int CH, int W, bool HAS_SEQ, int WM>
 int launch_instance(const cc1d_bwd_params &p, const BwdClGeom &g, float *ws, hipStream_t stream) {
     constexpr int U = CC1D_BWD_CL_UNROLL;
     const uint32_t blocks = g.blocks_per_xcd * kXcds;
-    if (p.silu)
-        CC1D_LAUNCH((bwd_channellast_kernel<DT, CH, W, HAS_SEQ, true, U, WM>), dim3(blocks), dim3(kBlock), 0, stream, p, g, ws, p.seq_idx);
-    else
-        CC1D_LAUNCH((bwd_channellast_kernel<DT, CH, W, HAS_SEQ, false, U, WM>), dim3(blocks), dim3(kBlock), 0, stream, p, g, ws, p.seq_idx);
+    if (!p.silu) {
+        CC1D_LAUNCH((bwd_channellast_kernel<DT, CH, W, HAS_SEQ, false, U, WM, false>), dim3(blocks), dim3(kBlock), 0, stream, p, g, ws, p.seq_idx);
+        return launch_status();
+    }
+    if constexpr (DT == CC1D_F16 && CH == 2 && HAS_SEQ && W == 4) {
+        if (takes_resources(p, g)) {
+            CC1D_LAUNCH((bwd_channellast_kernel<DT, CH, W, HAS_SEQ, true, U, WM, true>), dim3(blocks), dim3(kBlock), 0, stream, p, g, ws, p.seq_idx);
+            return launch_status();
+        }
+    }
+    CC1D_LAUNCH((bwd_channellast_kernel<DT, CH, W, HAS_SEQ, true, U, WM, false>), dim3(blocks), dim3(kBlock), 0, stream, p, g, ws, p.seq_idx);
     return launch_status();
 }
 
