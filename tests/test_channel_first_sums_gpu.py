@@ -18,6 +18,8 @@ BF16, FP16, FP32 = torch.bfloat16, torch.float16, torch.float32
 CASES = [   # batch, dim, seqlen, width, dtype, weight dtype, strided weight, (dim, batch, seqlen) in memory
     (1, 24, 513, 4, BF16, FP32, False, False),         # one tile of one step and a tail
     (2, 24, 2049, 4, FP16, FP16, False, False),        # two tiles, the second a tail only
+    (1, 17, 601, 4, BF16, BF16, False, False),         # channels by twos, the last one alone; rows off the dword grid
+    (2, 263, 1001, 4, FP16, FP32, False, False),
     (2, 16, 12000, 3, BF16, BF16, True, False),        # 12 tiles of four steps
     (14, 16, 1537, 4, BF16, BF16, False, False),       # 14 tiles of four steps: 61 KiB of LDS
     (15, 16, 1990, 4, BF16, FP32, False, False),       # 15 of them: one more than fit
