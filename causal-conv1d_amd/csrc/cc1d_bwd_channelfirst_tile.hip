@@ -453,19 +453,29 @@ int bwd_channelfirst_tile_parts(const cc1d_bwd_params &p) { return (int)(p.batch
 
 // Whether the kernel adds up the sums of a channel's tiles itself (DIRECT) instead of leaving them
 // to a second launch.  One workgroup must hold them all (its wavefronts, 64 KiB of LDS), and what the
-// second launch costs (2-3 us) must be more than what the other order of the tiles does: a
-// workgroup then reads and writes as many places as there are batch entries, where otherwise the launch
-// moves through memory as one front in the order of the rows.  Two places cost nothing; more of them
-// are worth it up to 8192 wavefronts.  Second stage / direct, us: (2, 64, 512) fp32 5.8 / 3.5,
-// (1, 5376, 2048) bf16 18.5 / 15.7, (1, 8192, 8192) 69.5 / 65.3, (2, 5376, 8192) fp16 88.9 / 86.8,
-// (8, 1024, 1024) bf16 15.2 / 13.2, (4, 2048, 1001) 16.1 / 15.4, (4, 2048, 2048) 23.1 / 23.3, and beyond the line
-// (4, 4096, 1001) 25.4 / 25.8, (8, 2048, 1024) 23.1 / 25.2, (4, 4096, 2048) 39.9 / 42.6.
+// second launch costs (2-3 us) must be more than what the other form of the launch does:
+//  * More than eight wavefronts to a workgroup leave wavefront slots empty where several workgroups
+//    share a CU, and the last round of workgroups leaves more CUs empty.  They pay while every workgroup has a
+//    CU of its own, if there are not so few that a CU's share is the launch.  Second launch / direct, us:
+//    (12, 256, 1528) bf16 10.7 / 8.6, (14, 256, 2040) 14.4 / 12.2, (12, 64, 1016) 6.6 / 5.9, but
+//    (14, 64, 2040) 8.4 / 9.9, (12, 320, 2040) 14.4 / 15.4, (1, 4096, 28000) 119 / 159.
+//  * A workgroup reads and writes as many places as there are batch entries, where otherwise the launch moves
+//    through memory as one front in the order of the rows.  One place costs nothing, nor do a channel's rows
+//    that lie together, up to 65536 wavefronts: (1, 65536, 600) bf16 72.3 / 59.8, (1, 8192, 8192) 69.5 / 65.3,
+//    and (4, 5376, 2048) of (dim, batch, seqlen) order 48.1 / 44.8, (8, 16384, 552) 93.8 / 96.6.  Two places cost little
+//    with up to two tiles to a row ((2, 5376, 4096) 48.3 / 46.1, (2, 5376, 5627) 69.2 / 71.3 with three), and more
+//    are worth it up to 8192 wavefronts: (8, 1024, 1024) 15.2 / 13.2, (4, 2048, 1001) 16.1 / 15.4, beyond them
+//    (8, 2048, 1024) 23.1 / 25.2, (4, 4096, 2048) 39.9 / 42.6.
 bool bwd_channelfirst_tile_direct(const cc1d_bwd_params &p) {
     const int64_t tiles = (int64_t)p.batch * tiles_per_row(p);
     if (tunables().bwd_cf_direct < 0 || tiles > kMaxDirectTiles || (size_t)tiles * tile_lds_bytes(steps_per_tile(p), p.width) > 64 * 1024)
         return false;
-    const bool adjacent = p.batch <= 2 || (p.dim > 1 && p.x_stride_b < p.x_stride_c);   // a channel's rows lie together
-    return adjacent || (int64_t)p.dim * tiles <= 8192;
+    constexpr int kCus = 256;
+    if (tiles > 8) return p.dim <= kCus && (p.dim >= 96 || tiles * steps_per_tile(p) <= 24);
+    if (p.batch == 1) return true;
+    const bool adjacent = p.dim > 1 && p.x_stride_b < p.x_stride_c;          // a channel's rows lie together
+    const int64_t most = adjacent ? 65536 : p.batch == 2 && tiles <= 4 ? 32767 : 8192;
+    return p.dim * tiles <= most;
 }
 
 bool bwd_channelfirst_tile_fits(const cc1d_bwd_params &p) {

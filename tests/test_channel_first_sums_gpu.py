@@ -1,8 +1,8 @@
-"""dweight / dbias of the channel-first kernels at the edges of the rule that picks who adds up a
-channel's tiles: the kernel's own workgroup (at most 16 tiles and 64 KiB of LDS, and at most two
-batch entries, a channel's rows adjacent in memory, or 8192 wavefronts; rows of at most 64 vectors: 2 to 16
-parts) or the second launch (`bwd_cf_direct` = -1 forces it).  dx and dinitial_states must not depend on it; dweight and dbias are the
-same fp32 terms added in another order.  Taps of every type, packed and strided."""
+"""dweight / dbias of the channel-first kernels at the edges of the rules that pick who adds up a
+channel's tiles: the kernel's own workgroup (`own`) or the second launch (`second`; `bwd_cf_direct` = -1
+forces it).  Which of the two ran shows in the workspace, which only the second launch's first stage writes.  dx and
+dinitial_states must not depend on it; dweight and dbias are the same fp32 terms added in another order.  Taps of
+every type, packed and strided."""
 import ctypes
 
 import pytest
@@ -15,33 +15,43 @@ from helpers import TOL_W, assert_close, gen, make_states
 pytestmark = pytest.mark.gpu
 
 BF16, FP16, FP32 = torch.bfloat16, torch.float16, torch.float32
-CASES = [   # batch, dim, seqlen, width, dtype, weight dtype, strided weight, (dim, batch, seqlen) in memory
-    (1, 24, 513, 4, BF16, FP32, False, False),         # one tile of one step and a tail
-    (2, 24, 2049, 4, FP16, FP16, False, False),        # two tiles, the second a tail only
-    (1, 17, 601, 4, BF16, BF16, False, False),         # channels by twos, the last one alone; rows off the dword grid
-    (2, 263, 1001, 4, FP16, FP32, False, False),
-    (2, 16, 12000, 3, BF16, BF16, True, False),        # 12 tiles of four steps
-    (14, 16, 1537, 4, BF16, BF16, False, False),       # 14 tiles of four steps: 61 KiB of LDS
-    (15, 16, 1990, 4, BF16, FP32, False, False),       # 15 of them: one more than fit
-    (16, 16, 1001, 2, FP32, FP32, True, False),        # 16 tiles
-    (17, 16, 600, 4, BF16, FP16, False, False),        # 17
-    (8, 1024, 520, 4, BF16, FP32, False, False),       # 8192 wavefronts
-    (8, 1032, 520, 4, BF16, FP32, False, False),       # 8256
-    (8, 1032, 520, 4, BF16, FP32, False, True),        # a channel's rows adjacent: any number
-    (1, 24, 512, 4, BF16, FP32, False, False),         # short rows: one part
-    (2, 24, 512, 4, BF16, BF16, False, False),         # two parts
-    (16, 24, 505, 3, FP16, FP32, True, False),         # 16, rows off the vector grid
-    (17, 24, 256, 4, FP32, FP32, False, False),        # 17
-    (64, 24, 60, 2, BF16, FP32, False, False),         # eight rows to a wavefront, eight parts
-    (100, 24, 1, 4, FP32, FP32, False, False),         # rows of one element, two parts
-    (5, 1500, 100, 4, FP16, FP16, False, True),        # parts of several wavefronts' rows
+CASES = [   # batch, dim, seqlen, width, dtype, weight dtype, strided weight, (dim, batch, seqlen) in memory, who adds
+    (1, 24, 513, 4, BF16, FP32, False, False, "own"),        # one tile of one step and a tail
+    (2, 24, 2049, 4, FP16, FP16, False, False, "own"),       # two tiles, the second a tail only
+    (1, 17, 601, 4, BF16, BF16, False, False, "own"),        # channels by twos, the last one alone; rows off the dword grid
+    (2, 263, 1001, 4, FP16, FP32, False, False, "own"),
+    (2, 16, 12000, 3, BF16, BF16, True, False, "second"),    # 12 tiles of four steps, few channels
+    (12, 95, 1001, 4, BF16, FP32, False, False, "own"),      # 12 of two steps
+    (9, 95, 1100, 4, BF16, FP32, False, False, "second"),    # 9 of three
+    (9, 96, 1100, 4, BF16, FP32, False, False, "own"),
+    (9, 256, 600, 4, BF16, FP16, False, False, "own"),       # as many channels as CUs
+    (9, 257, 600, 4, BF16, FP16, False, False, "second"),
+    (14, 96, 1990, 4, BF16, BF16, False, False, "own"),      # 14 of four steps: 61,656 bytes of LDS
+    (15, 96, 1990, 4, BF16, FP32, False, False, "second"),   # 15 of them: more than 64 KiB
+    (16, 96, 1001, 2, BF16, FP32, True, False, "own"),       # 16 wavefronts
+    (16, 96, 505, 4, FP32, FP32, False, False, "own"),
+    (16, 96, 1001, 2, FP32, FP32, True, False, "second"),    # 16 of four steps: more than 64 KiB
+    (17, 96, 600, 4, BF16, FP16, False, False, "second"),    # 17
+    (8, 1024, 520, 4, BF16, FP32, False, False, "own"),      # 8192 wavefronts
+    (8, 1032, 520, 4, BF16, FP32, False, False, "second"),   # 8256
+    (8, 1032, 520, 4, BF16, FP32, False, True, "own"),       # a channel's rows adjacent
+    (2, 4200, 520, 4, BF16, FP32, False, False, "own"),      # two places, one tile to a row: 8400 wavefronts
+    (2, 1366, 4200, 4, BF16, FP32, False, False, "second"),  # three tiles to a row: 8196
+    (1, 24, 512, 4, BF16, FP32, False, False, "one part"),   # short rows
+    (2, 24, 512, 4, BF16, BF16, False, False, "own"),        # two parts
+    (16, 24, 505, 3, FP16, FP32, True, False, "own"),        # 16, rows off the vector grid
+    (17, 24, 256, 4, FP32, FP32, False, False, "second"),    # 17
+    (64, 24, 60, 2, BF16, FP32, False, False, "own"),        # eight rows to a wavefront, eight parts
+    (100, 24, 1, 4, FP32, FP32, False, False, "own"),        # rows of one element, two parts
+    (5, 1500, 100, 4, FP16, FP16, False, True, "own"),       # parts of several wavefronts' rows
 ]
 
 
+@pytest.mark.parametrize("has_bias", [True, False], ids=["bias", "no_bias"])
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(v).replace("torch.", "") for v in c))
-def test_sums_do_not_depend_on_who_adds_them(gpu_device, cc1d_lib, case):
+def test_sums_do_not_depend_on_who_adds_them(gpu_device, cc1d_lib, case, has_bias):
     lib, dev = cabi.declare(cc1d_lib), gpu_device
-    B, D, L, W, dtype, wtype, strided, batch_inner = case
+    B, D, L, W, dtype, wtype, strided, batch_inner, who = case
     g = gen(B * 1000 + L)
 
     def tensor():
@@ -53,7 +63,7 @@ def test_sums_do_not_depend_on_who_adds_them(gpu_device, cc1d_lib, case):
     w = w[:, ::2] if strided else w
     b = (torch.rand(D, generator=g) - 0.5).to(wtype)
     init, dfin = make_states(B, D, W - 1, dtype, g), make_states(B, D, W - 1, dtype, g)
-    xd, dd, bd, initd, dfind = x.to(dev), dout.to(dev), b.to(dev), init.to(dev), dfin.to(dev)
+    xd, dd, bd, initd, dfind = x.to(dev), dout.to(dev), b.to(dev) if has_bias else None, init.to(dev), dfin.to(dev)
     wd = torch.empty(D, 2 * W, dtype=wtype, device=dev)[:, ::2] if strided else torch.empty(D, W, dtype=wtype, device=dev)
     wd.copy_(w)
 
@@ -63,20 +73,23 @@ def test_sums_do_not_depend_on_who_adds_them(gpu_device, cc1d_lib, case):
         dw, db = torch.full((D, W), float("nan"), device=dev), torch.full((D,), float("nan"), device=dev)
         got = []
         for overwrite in (1, 0):                        # stored, then the same once more on top
-            p = cabi.bwd_params(xd, wd, bd, dd, dx, dw, db, True, initial_states=initd, dfinal_states=dfind,
+            p = cabi.bwd_params(xd, wd, bd, dd, dx, dw, db if has_bias else None, True, initial_states=initd, dfinal_states=dfind,
                                 dinitial_states=dinit)
             p.overwrite_dweight = overwrite
             assert lib.cc1d_set_tunable(b"bwd_cf_direct", knob) == 0
             try:
                 need = ctypes.c_size_t()
                 assert lib.cc1d_bwd_workspace_bytes(ctypes.byref(p), ctypes.byref(need)) == 0
-                ws = torch.empty(max(16, need.value), dtype=torch.uint8, device=dev)
+                ws = torch.full((max(16, need.value),), 0xA5, dtype=torch.uint8, device=dev)
                 stream = torch.cuda.current_stream().cuda_stream
                 assert lib.cc1d_bwd(ctypes.byref(p), ws.data_ptr(), need.value, stream) == 0
                 torch.cuda.synchronize()
             finally:
                 lib.cc1d_set_tunable(b"bwd_cf_direct", 0)
-            got += [dw.clone(), db.clone()]
+            assert (need.value == 0) == (who == "one part")
+            assert bool((ws == 0xA5).all()) == (who == "one part" or (who == "own" and knob == 0))
+            assert has_bias or bool(db.isnan().all())
+            got += [dw.clone(), db.clone()] if has_bias else [dw.clone()] * 2
         return [dx, dinit] + got
 
     own, second = run(0), run(-1)
@@ -87,9 +100,10 @@ def test_sums_do_not_depend_on_who_adds_them(gpu_device, cc1d_lib, case):
     terms = 1.1 * dout.float().abs().sum((0, 2)) * x.float().abs().amax((0, 2)).clamp(min=1.0)
     bound = (2 * 55 * 2.0 ** -24 * terms).to(dev)
     assert bool(((own[2] - second[2]).abs() <= bound[:, None]).all())
-    assert bool(((own[3] - second[3]).abs() <= bound).all())
-    rdx, rdw, rdb, rdi = orc.bwd(x, w.float().contiguous(), b.float(), dout, initial_states=init, dfinal_states=dfin, activation="silu")
+    rdx, rdw, rdb, rdi = orc.bwd(x, w.float().contiguous(), b.float() if has_bias else None, dout, initial_states=init, dfinal_states=dfin, activation="silu")
     assert_close(own[0], rdx, dtype, "dx")
     assert_close(own[1], rdi, dtype, "dinitial_states")
     assert_close(own[2], rdw, what="dweight", tol=TOL_W)
-    assert_close(own[3], rdb, what="dbias", tol=TOL_W)
+    if has_bias:
+        assert bool(((own[3] - second[3]).abs() <= bound).all())
+        assert_close(own[3], rdb, what="dbias", tol=TOL_W)
