@@ -670,9 +670,8 @@ constexpr int kMaxDirectParts = 16;
 // and written element by element (positions past the row's end read as zero).
 // DIRECT: the parts of a channel, two to sixteen, are the wavefronts of one workgroup, which adds up
 // their sums and stores dweight / dbias itself.  The wavefronts take the same rows in the same order as
-// without it; what goes is the second launch, 2-5 us behind a kernel that may run for less.  Two launches /
-// one, us: (4, 1024, 300) bf16 11.3 / 8.7, (16, 512, 256) 8.2 / 6.0, (32, 256, 64) 6.5 / 4.3, (16, 1024, 505)
-// 36.2 / 33.5, (32, 2048, 512) 43.2 / 40.0, (2, 64, 128) fp32 3.6 / 3.5: never slower.
+// without it; what goes is the second launch, 2-5 us behind a kernel that may run for less (see
+// short_rows_direct for where that is worth it).
 template <int DT, int W, bool ALIGNED, bool DIRECT>
 __global__ void __launch_bounds__(DIRECT ? kMaxDirectParts * kWave : kBlock)
 bwd_channelfirst_short_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float *__restrict__ ws) {
@@ -947,14 +946,40 @@ BwdCfGeom make_geom(const cc1d_bwd_params &p) {
     return g;
 }
 
-// Short rows whose kernel adds up a channel's parts itself (see DIRECT).
-bool short_rows_direct(const BwdCfGeom &g) {
-    return (g.streaming == 3 || g.streaming == 4) && g.n_parts > 1 && g.n_parts <= kMaxDirectParts && tunables().bwd_cf_direct >= 0;
+// Short rows whose kernel adds up a channel's parts itself (see DIRECT).  What the second launch costs
+// stays the same, what the other form costs grows with the launch:
+//  * A workgroup's wavefronts must find room on one CU together and hold it until the last of them ends.  The
+//    kernels take 49-75 registers, and 80-93 for 16-bit rows off the vector grid, five to eight wavefronts a
+//    SIMD; 13 to 16 to a workgroup then leave up to half of the slots empty, 9 to 12 and 5 to 8 fewer.  So
+//    large workgroups only where each has a CU of its own (256 channels) or enough of them fit, and few items
+//    to a wavefront, one after the other.
+//  * Channels whose rows share cache lines go to different XCDs, where two or three parts leave room for another
+//    channel in a workgroup of four.  So two items at most there, and next to nothing of rows of a few dwords.
+// Two launches / one, us, parts x items: (4, 1024, 300) bf16 4 x 1 11.3 / 8.7, (32, 256, 64) 4 x 1 6.5 / 4.3,
+// (8, 512, 512) 8 x 1 8.4 / 6.0, (8, 2048, 512) 2 x 4 15.6 / 12.7, (80, 410, 64) 10 x 1 8.3 / 6.4, (16, 256, 509) 16 x 1
+// 13.0 / 10.8, but (14, 300, 512) 14 x 1 8.6 / 9.1, (16, 64, 509) 8.1 / 8.8, (18, 818, 512) 6 x 3 13.8 / 14.3,
+// (32, 4095, 61) 2 x 2 39.1 / 40.1, (96, 683, 509) 6 x 16 131 / 195, (224, 300, 512) 14 x 16 48.9 / 67.1,
+// (256, 256, 512) 16 x 16 41.7 / 45.3, and for the lines (240, 2048, 16) 2 x 4 32.9 / 44.9, (124, 2048, 48) 2 x 8 28.0 / 36.1,
+// (992, 64, 8) 16 x 1 8.4 / 14.7.
+bool short_rows_direct(const cc1d_bwd_params &p, const BwdCfGeom &g) {
+    if ((g.streaming != 3 && g.streaming != 4) || g.n_parts <= 1 || tunables().bwd_cf_direct < 0) return false;
+    constexpr int kCus = 256, kLine = 128;
+    const int eb = elem_bytes(p.x_dtype);
+    if ((int64_t)p.seqlen * eb < kLine / 2) return g.n_parts <= 4 && g.items_per_part == 1 && p.dim <= 3 * kCus;
+    const bool aligned = g.streaming == 3;
+    const bool light = aligned || p.x_dtype == CC1D_F32;
+    const bool own_lines = p.x_stride_c * eb % kLine == 0;
+    int most_parts, most_items;
+    if (p.dim <= kCus) most_parts = light || p.dim >= kCus / 2 ? kMaxDirectParts : 12;
+    else most_parts = light ? 12 : p.dim <= 2 * kCus ? 8 : 4;
+    if (!aligned || (g.n_parts < 4 && !own_lines)) most_items = g.n_parts <= 8 && p.dim <= 8 * kCus ? 2 : 1;
+    else most_items = g.n_parts <= 4 ? 6 : p.dim <= kCus ? 4 : g.n_parts <= 8 && p.dim <= 3 * kCus ? 3 : 2;
+    return g.n_parts <= most_parts && g.items_per_part <= most_items;
 }
 
 template <int DT, bool ALIGNED>
 int launch_short(const cc1d_bwd_params &p, const BwdCfGeom &g, float *ws, hipStream_t stream) {
-    const bool direct = short_rows_direct(g);
+    const bool direct = short_rows_direct(p, g);
     const uint32_t waves = direct ? (uint32_t)g.n_parts : (uint32_t)(kBlock / kWave);
     const uint32_t blocks = (uint32_t)(((int64_t)p.dim * g.n_parts + waves - 1) / waves);
     auto launch = [&](auto width) {
@@ -1035,7 +1060,7 @@ int launch_bwd_channelfirst(const cc1d_bwd_params &p, void *workspace, hipStream
         case CC1D_F16: st = launch_dtype<CC1D_F16>(p, g, ws, stream); break;
         default: st = launch_dtype<CC1D_BF16>(p, g, ws, stream); break;
     }
-    if (st != CC1D_OK || g.n_parts == 1 || short_rows_direct(g)) return st;   // the kernel wrote dweight / dbias itself
+    if (st != CC1D_OK || g.n_parts == 1 || short_rows_direct(p, g)) return st;   // the kernel wrote dweight / dbias itself
     return launch_bwd_finalize(ws, g.n_parts, p, stream);
 }
 

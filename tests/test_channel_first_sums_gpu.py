@@ -37,13 +37,48 @@ CASES = [   # batch, dim, seqlen, width, dtype, weight dtype, strided weight, (d
     (8, 1032, 520, 4, BF16, FP32, False, True, "own"),       # a channel's rows adjacent
     (2, 4200, 520, 4, BF16, FP32, False, False, "own"),      # two places, one tile to a row: 8400 wavefronts
     (2, 1366, 4200, 4, BF16, FP32, False, False, "second"),  # three tiles to a row: 8196
-    (1, 24, 512, 4, BF16, FP32, False, False, "one part"),   # short rows
-    (2, 24, 512, 4, BF16, BF16, False, False, "own"),        # two parts
-    (16, 24, 505, 3, FP16, FP32, True, False, "own"),        # 16, rows off the vector grid
-    (17, 24, 256, 4, FP32, FP32, False, False, "second"),    # 17
-    (64, 24, 60, 2, BF16, FP32, False, False, "own"),        # eight rows to a wavefront, eight parts
-    (100, 24, 1, 4, FP32, FP32, False, False, "own"),        # rows of one element, two parts
-    (5, 1500, 100, 4, FP16, FP16, False, True, "own"),       # parts of several wavefronts' rows
+    # short rows; parts of a channel x items of a part
+    (1, 24, 512, 4, BF16, FP32, False, False, "one part"),
+    (2, 24, 512, 4, BF16, BF16, False, False, "own"),        # 2 x 1
+    (16, 24, 512, 4, FP16, FP16, False, False, "own"),       # 16 x 1
+    (17, 24, 256, 4, FP32, FP32, False, False, "second"),    # 17 x 1
+    (256, 256, 64, 4, FP32, FP32, False, False, "own"),      # 16 x 4, as many channels as CUs
+    (260, 256, 64, 4, FP32, FP32, False, False, "second"),   # 13 x 5
+    (48, 257, 64, 4, FP32, BF16, True, False, "own"),        # 12 x 1, more channels
+    (52, 257, 64, 4, FP32, FP32, False, False, "second"),    # 13 x 1
+    (72, 700, 64, 3, FP32, FP32, False, False, "own"),       # 6 x 3
+    (76, 700, 64, 3, FP32, FP32, False, False, "second"),    # 5 x 4
+    (48, 800, 64, 4, FP32, FP32, False, False, "own"),       # 6 x 2
+    (52, 800, 64, 4, FP32, FP32, False, False, "second"),    # 5 x 3
+    (96, 2048, 32, 2, FP32, FP32, False, False, "own"),      # 2 x 6, rows of a cache line each
+    (104, 2048, 32, 2, FP32, FP32, False, False, "second"),  # 2 x 7
+    (32, 2048, 40, 4, BF16, FP32, False, False, "own"),      # 2 x 2, rows that share cache lines
+    (40, 2048, 40, 4, BF16, FP32, False, False, "second"),   # 2 x 3
+    (32, 2056, 40, 4, BF16, FP32, False, False, "second"),   # 2 x 2, 8 x 256 channels and more
+    (80, 24, 32, 4, BF16, FP32, False, False, "own"),        # 5 x 1, rows of 64 bytes
+    (80, 24, 31, 4, BF16, FP32, False, False, "second"),     # 62 bytes
+    (64, 24, 31, 4, BF16, FP32, False, False, "own"),        # 4 x 1
+    (65, 256, 8, 3, BF16, BF16, False, False, "own"),        # 2 x 1
+    (320, 1024, 8, 3, BF16, BF16, False, False, "second"),   # 3 x 2
+    (65, 768, 8, 3, BF16, BF16, False, False, "own"),        # 2 x 1
+    (65, 776, 8, 3, BF16, BF16, False, False, "second"),
+    (12, 24, 505, 3, FP16, FP32, True, False, "own"),        # 16-bit rows off the vector grid: 12 x 1, few channels
+    (16, 24, 505, 3, FP16, FP32, True, False, "second"),     # 16 x 1
+    (16, 128, 505, 3, FP16, FP32, True, False, "own"),
+    (64, 512, 61, 4, BF16, FP32, False, False, "own"),       # 8 x 1
+    (64, 513, 61, 4, BF16, FP32, False, False, "second"),
+    (32, 513, 61, 4, BF16, FP32, False, False, "own"),       # 4 x 1
+    (16, 24, 253, 4, FP32, FP32, False, False, "own"),       # fp32 rows off the vector grid: 16 x 1, few channels
+    (56, 600, 61, 4, FP32, FP32, False, False, "own"),       # 7 x 2
+    (60, 600, 61, 4, FP32, FP32, False, False, "second"),    # 5 x 3
+    (32, 2049, 61, 4, BF16, FP32, False, False, "second"),   # 2 x 2, 8 x 256 channels and one more
+    (88, 400, 64, 4, FP32, FP32, False, False, "own"),       # 11 x 2
+    (132, 400, 64, 4, FP32, FP32, False, False, "second"),   # 11 x 3
+    (44, 400, 61, 4, FP32, FP16, False, False, "own"),       # 11 x 1
+    (88, 400, 61, 4, FP32, FP16, False, False, "second"),    # 11 x 2
+    (64, 24, 60, 2, BF16, FP32, False, False, "own"),        # eight rows to a wavefront, 8 x 1
+    (100, 24, 1, 4, FP32, FP32, False, False, "own"),        # rows of one element, 2 x 1
+    (5, 1500, 100, 4, FP16, FP16, False, True, "own"),       # a channel's rows adjacent, 2 x 1
 ]
 
 
