@@ -58,6 +58,63 @@ def test_left_to_the_generic_path(pkg):
     assert pkg.causal_conv1d_fn(x.to("meta"), w.to("meta")).shape == x.shape
 
 
+def _backward_args():
+    return [torch.zeros(2, 8, 9), torch.zeros(8, 4), torch.zeros(8), torch.zeros(2, 8, 9), torch.zeros(2, 9, dtype=torch.int32),
+            torch.zeros(2, 8, 3), torch.zeros(2, 8, 3), True, True]
+
+
+def test_backward_left_to_the_generic_path(pkg):
+    import causal_conv1d_cuda as ext
+    for i in range(9):
+        a = _backward_args()
+        if i < 7:
+            a[i] = a[i].as_subclass(_Subclass)
+            assert ext._backward_call(*a) is NotImplemented
+        for other in ((5,) if i in (2, 4, 5, 6) else (5, None)):
+            a[i] = other
+            assert ext._backward_call(*a) is NotImplemented
+    assert ext._backward_call(*_backward_args()[:-1]) is NotImplemented
+    for i, t in ((0, torch.zeros(8, 9)), (1, torch.zeros(8, 1, 4)), (3, torch.zeros(2, 16, 18)[:, ::2, ::2])):
+        a = _backward_args()
+        a[i] = t                                                    # x not (batch, dim, seqlen), weight not (dim, width), dout needs a copy
+        assert ext._backward_call(*a) is NotImplemented
+    with _Functions():
+        assert ext._backward_call(*_backward_args()) is NotImplemented
+    with pytest.raises(RuntimeError, match="must be on the GPU"):
+        ext._backward_call(*_backward_args())
+
+
+@pytest.mark.filterwarnings("ignore:.*torch.jit.trace")
+def test_tracing_sees_the_ops(pkg):
+    """On meta tensors: the direct calls step aside while torch.jit.trace records."""
+    import causal_conv1d_cuda as ext
+    answers = []
+
+    def step(x, st):
+        answers.append(ext._update_call(x, st, w, None, True, None, None))
+        answers.append(ext._forward_call(st, w, None, None, None, False, None, True))
+        answers.append(ext._backward_call(st, w, None, st, None, None, None, False, True))
+        return pkg.causal_conv1d_update(x, st, w)
+
+    w = torch.zeros(8, 4, device="meta")
+    traced = torch.jit.trace(step, (torch.zeros(2, 8, device="meta"), torch.zeros(2, 8, 4, device="meta")), check_trace=False)
+    assert len(answers) == 3 and all(a is NotImplemented for a in answers)
+    assert "DaoAILab::_causal_conv1d_update_out_cpp" in str(traced.graph)
+
+
+def test_vmap_is_refused_by_both_ways(pkg, monkeypatch):
+    """The ops have no batching rule; the direct calls reach the dispatcher with the same batched tensors."""
+    from causal_conv1d import causal_conv1d_interface as interface
+    x, w, st = torch.zeros(3, 2, 8, device="meta"), torch.zeros(8, 4, device="meta"), torch.zeros(3, 2, 8, 4, device="meta")
+    for _ in range(2):
+        with pytest.raises(RuntimeError, match="Batching rule not implemented for DaoAILab::_causal_conv1d_update_out_cpp"):
+            torch.vmap(lambda q, s: pkg.causal_conv1d_update(q, s, w))(x, st)
+        with pytest.raises(RuntimeError, match="Batching rule not implemented for DaoAILab::_causal_conv1d_fwd_out_cpp"):
+            torch.vmap(lambda q: pkg.causal_conv1d_fn(q, w))(st)
+        monkeypatch.setattr(interface, "_direct_update", lambda *a: NotImplemented)
+        monkeypatch.setattr(interface, "_direct_forward", lambda *a: NotImplemented)
+
+
 def test_dispatch_modes_see_the_ops(pkg):
     """On meta tensors, without a GPU."""
     x, w, st = torch.zeros(2, 8, device="meta"), torch.zeros(8, 4, device="meta"), torch.zeros(2, 8, 4, device="meta")
@@ -72,9 +129,24 @@ def test_dispatch_modes_see_the_ops(pkg):
 @pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: str(d)[6:])
 @pytest.mark.parametrize("channel_last", [False, True], ids=["cf", "cl"])
 @pytest.mark.parametrize("extra", ["none", "states", "seq_idx", "no_bias"])
-def test_both_paths_give_the_same(pkg, gpu_device, channel_last, dtype, extra, wide_weights):
+def test_both_paths_give_the_same(pkg, gpu_device, monkeypatch, channel_last, dtype, extra, wide_weights):
     if extra == "seq_idx" and not channel_last:
         pytest.skip("seq_idx needs channel-last x")
+    from causal_conv1d import causal_conv1d_interface as interface, cpp_functions
+    answers = {}
+
+    def watched(module, name):
+        call = getattr(module, name)
+
+        def wrapper(*args):
+            res = call(*args)
+            answers.setdefault(name, []).append(res is not NotImplemented)
+            return res
+        monkeypatch.setattr(module, name, wrapper)
+
+    watched(interface, "_direct_forward")
+    watched(interface, "_direct_update")
+    watched(cpp_functions, "_direct_backward")
     g = gen(31)
     B, D, L, W = 2, 40, 77, 4
     wtype = torch.float32 if wide_weights else dtype
@@ -102,8 +174,12 @@ def test_both_paths_give_the_same(pkg, gpu_device, channel_last, dtype, extra, w
         return outs + list(grads) + (list(quiet) if isinstance(quiet, tuple) else [quiet]) + [st, step]
 
     direct = everything()
-    with _Functions():                                              # every call takes torch.ops
+    calls = {"_direct_forward": 2, "_direct_backward": 1, "_direct_update": 1}
+    assert answers == {name: [True] * n for name, n in calls.items()}
+    answers.clear()
+    with _Functions():                                              # every call takes torch.ops, the engine's thread included
         generic = everything()
+    assert answers == {name: [False] * n for name, n in calls.items()}
     assert len(direct) == len(generic)
     for d, r in zip(direct, generic):
         assert d.dtype == r.dtype and d.stride() == r.stride() and torch.equal(d, r)
