@@ -3,7 +3,7 @@
 microseconds per call, achieved GB/s against the bytes the operator must move, and peak
 device memory.  The role of tests/benchmark_determinism_kernels.py in the reference, for
 all four operators; there is no deterministic/non-deterministic pair to compare because the
-backward here is always a fixed-order two-stage sum.
+backward here always adds in a fixed order.
 
   python benchmark_ops.py --op fwd --batch 8 --dim 5376 --seqlen 2048 --channel-last --seq-idx
   python benchmark_ops.py --op bwd --batch 4 --dim 4096 --seqlen 8192 --dtype fp16 --states

@@ -6,8 +6,9 @@
 //
 // This file is host-only C++ (built with g++, no device code, no source translation):
 // it checks tensors, fills the C-ABI parameter blocks of include/cc1d.h, takes the
-// current HIP stream from c10 and calls the kernel library.  The only memory it
-// allocates is the backward workspace, through the caching allocator.
+// current HIP stream from c10 and calls the kernel library.  The entry points above allocate
+// nothing but the backward workspace; the ops that return their result (`*_out`) and the direct
+// calls below allocate that too, all through the caching allocator.
 #include <torch/extension.h>
 #include <torch/library.h>
 #include <torch/csrc/Exceptions.h>
@@ -476,7 +477,8 @@ void update_meta(const at::Tensor &, at::Tensor &, const at::Tensor &, const std
 // ops, called with plain C++ arguments.  What is left out is the generic parsing of Python arguments
 // against the op's schema into a stack of boxed values and back: 1.1 instead of 2.0 us of host time for
 // a decode call without its launch.  32 layers of one request, which the host bounds: 178 -> 149 us,
-// uninitialised_like included.  Everything behind the dispatcher (autograd's handling, fake tensors, dispatch modes, profiling) sees the same call.
+// uninitialised_like included.  Everything behind the dispatcher (autograd's handling, fake tensors, dispatch
+// modes, profiling) sees the same call.
 // Each returns NotImplemented, having done nothing, for what the generic path in Python has to
 // handle: tensor subclasses, torch-function modes, tracing, arguments of other types or that still need a copy.
 

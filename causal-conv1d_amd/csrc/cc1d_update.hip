@@ -284,7 +284,9 @@ update_step_kernel(const StepArgs a) {
     Staging staging;
     staging.request(a.weight, a.bias, col0, cols_here);
 
-    // Everything this lane reads is requested up front.
+    // Everything this lane reads is requested before any of it is used.  Where a row's slot and position are
+    // read too (conv_state_indices, cache_seqlens), its state rows wait for the two, one after the other, and
+    // the next row's slot for them: four round trips in front of the last request with two rows to a lane.
     raw_t rw[R][W - 1], xr[R];
     int64_t soff[R];
     int wpos[R];

@@ -112,14 +112,16 @@ int cc1d_fwd(const cc1d_fwd_params *p, cc1d_stream_t stream);
  * dweight (fp32, (dim, width)) and dbias (fp32, (dim,)) are ACCUMULATED INTO, like the
  * reference (atomicAdd at bwd.cu:243,255 / add_ at causal_conv1d.cpp:452-459): the
  * caller zeroes them first.  With overwrite_dweight = 1 they are plain outputs instead and
- * need no zeroing (two fill launches fewer per backward call).  The reduction is always a
- * fixed-order two-stage sum (partials in the workspace, then one ordered pass), so results are
+ * need no zeroing (two fill launches fewer per backward call).  The reduction always adds
+ * partial sums in a fixed order, either in a second launch (partials in the workspace) or, for some
+ * channel-first launches, in the workgroup that holds all of a channel, so results are
  * bit-reproducible run to run; the reference's `deterministic` switch
  * (causal_conv1d.cpp:21-28, 388-437) has nothing left to select.
  *
  * The workspace is caller-owned device memory, 16-byte aligned, of at least
  * cc1d_bwd_workspace_bytes() bytes (the reference allocates its own with at::zeros,
- * causal_conv1d.cpp:396-429).  It needs no initialisation.  A problem too large for one grid is
+ * causal_conv1d.cpp:396-429).  It needs no initialisation, and is asked for also where the launch that
+ * is picked leaves it untouched.  A problem too large for one grid is
  * launched as slices of the batch, one after the other on the stream, each adding into
  * dweight / dbias: the sums then follow the slice order (still the same bits run to run).
  * ---------------------------------------------------------------------------------- */
