@@ -100,8 +100,9 @@ __device__ __forceinline__ float wave_total_in_lane63(float v) {
 // traffic.  Otherwise the wavefronts are numbered along the rows, four to a workgroup, and leave their
 // sums to the second stage.  See bwd_channelfirst_tile_direct for the line between the two.
 // Registers: 64 at most (16-bit data), so that eight wavefronts share a SIMD; wave-uniform values
-// (taps, the odd last element, dfinal_states) live in scalar registers for that.  The launch is bound
-// by memory and by the vector ALUs about equally, and what counts is how well the two overlap:
+// (taps, the odd last element, dfinal_states) live in scalar registers for that.  The memory pattern
+// bounds the launch (without the activation's derivative, half of the arithmetic, fp16 (4, 4096, 8192)
+// takes 4 % less) as long as the arithmetic overlaps with it:
 // 65 registers and seven wavefronts measured (16, 4096, 1001) bf16 85.0 us against 80.8 now with 57
 // and eight, (16, 4096, 1024) 75.6 against 73.3, fp16 (4, 4096, 8192) 139.2 against 136.2 (second stage
 // included).
