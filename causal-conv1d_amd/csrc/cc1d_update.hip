@@ -40,9 +40,27 @@ __device__ __forceinline__ int wrap(int v, int n) {   // v in (-n, 2n) -> [0, n)
     return v >= n ? v - n : v;
 }
 __device__ __forceinline__ int positive_mod(int v, int n) {
+    if ((n & (n - 1)) == 0) return v & (n - 1);       // the usual ring, without the division's two dozen instructions
     const int r = v % n;
     return r < 0 ? r + n : r;
 }
+
+// Walks the positions of a wave-uniform row of conv_state one after the other: `off` is the position's
+// element offset, kept by additions (a 64-bit product of scalars takes five instructions, and a decode
+// step's wavefront has nothing else to do until its addresses are there).  RING: behind the last position
+// comes position 0.
+template <bool RING>
+struct Positions {
+    int64_t off;
+    int at;
+    __device__ __forceinline__ Positions(int first, int64_t stride) : off((int64_t)first * stride), at(first) {}
+    __device__ __forceinline__ void next(int64_t stride, int state_len) {
+        ++at;
+        const bool over = RING && at == state_len;
+        at = over ? 0 : at;
+        off = over ? 0 : off + stride;
+    }
+};
 
 template <int DT, int W, bool CIRC>
 __global__ void __launch_bounds__(kBlock)
@@ -275,39 +293,56 @@ update_step_kernel(const StepArgs a) {
     // Lanes past the last column group shadow the block's first one: every address they form
     // is valid, and they store nothing.
     const bool col_ok = lc < cols_here;
-    const int c0 = (int)(col0 + (col_ok ? lc : 0u)) * CH;
+    const uint32_t lane_bytes = (col_ok ? lc : 0u) * (uint32_t)sizeof(raw_t);
     const int S = a.state_len;
-    const T *xb = reinterpret_cast<const T *>(a.x);
-    T *ob = reinterpret_cast<T *>(a.out);
-    T *sbase = reinterpret_cast<T *>(a.conv_state);
+    // The block's columns of x, out and conv_state: every row is a scalar address plus the lane's bytes.
+    const T *xb = reinterpret_cast<const T *>(a.x) + (int64_t)col0 * CH;
+    T *ob = reinterpret_cast<T *>(a.out) + (int64_t)col0 * CH;
+    T *sbase = reinterpret_cast<T *>(a.conv_state) + (int64_t)col0 * CH;
+    auto lane_of = [&](const T *row) __attribute__((always_inline)) {
+        return reinterpret_cast<raw_t *>(const_cast<char *>(reinterpret_cast<const char *>(row)) + lane_bytes);
+    };
 
     Staging staging;
     staging.request(a.weight, a.bias, col0, cols_here);
 
-    // Everything this lane reads is requested before any of it is used.  Where a row's slot and position are
-    // read too (conv_state_indices, cache_seqlens), its state rows wait for the two, one after the other, and
-    // the next row's slot for them: four round trips in front of the last request with two rows to a lane.
+    // Everything this lane reads is requested before any of it is used: taps and x rows first, then the
+    // slots and positions of all its rows (conv_state_indices, cache_seqlens) in one round trip, which the
+    // state rows wait for.  Slot, position and state of one row after the other were four trips in a row:
+    // bf16 ring buffers (128, 5376, 8) in 512 slots 4.74 -> 4.46 us a launch, fp32 (64, 5376, 8) in 128 4.36 -> 3.88,
+    // (512, 2560, 16) in 1024 5.40 -> 5.03; without slots and rings 5.9 us as before at (256, 5376, 3).
     raw_t rw[R][W - 1], xr[R];
-    int64_t soff[R];
-    int wpos[R];
+    T *st[R];                                         // the row's state; RING: its position to be written
+    int srow[R], cs[R];
     bool live[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int b = ((int)blockIdx.y * kStepWaves + wave_row) * R + r;
         live[r] = b < a.batch;
-        const int bb = live[r] ? b : 0;
-        const int srow = a.conv_state_indices == nullptr ? bb : a.conv_state_indices[bb];
-        live[r] = live[r] && srow >= 0;
-        soff[r] = (int64_t)(srow < 0 ? 0 : srow) * a.state_stride_b + c0;
-        int cs = 0;
-        if (CIRC) cs = positive_mod(a.cache_seqlens[bb], S);
-        wpos[r] = cs;
+        srow[r] = live[r] ? b : 0;
+        cs[r] = CIRC ? a.cache_seqlens[srow[r]] : 0;
+        xr[r] = *lane_of(xb + (int64_t)srow[r] * a.x_stride_b);
+    }
+    if (a.conv_state_indices != nullptr) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) srow[r] = a.conv_state_indices[srow[r]];
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        live[r] = live[r] && srow[r] >= 0;
+        st[r] = sbase + (int64_t)(srow[r] < 0 ? 0 : srow[r]) * a.state_stride_b;
+        int first = S - (W - 1);
+        if (CIRC) {
+            first = positive_mod(cs[r], S) - (W - 1);
+            first = first < 0 ? first + S : first;
+        }
+        Positions<CIRC> pos(first, a.state_stride_l);
 #pragma unroll
         for (int i = 0; i < W - 1; ++i) {
-            const int l = CIRC ? wrap(cs - (W - 1) + i, S) : S - (W - 1) + i;
-            rw[r][i] = ld_state(reinterpret_cast<const raw_t *>(sbase + soff[r] + (int64_t)l * a.state_stride_l));
+            rw[r][i] = ld_state(lane_of(st[r] + pos.off));
+            pos.next(a.state_stride_l, S);
         }
-        xr[r] = *reinterpret_cast<const raw_t *>(xb + (int64_t)bb * a.x_stride_b + c0);
+        if (CIRC) st[r] += pos.off;
     }
 
     staging.publish(staged);
@@ -322,26 +357,27 @@ update_step_kernel(const StepArgs a) {
     for (int r = 0; r < R; ++r) {
         const int b = ((int)blockIdx.y * kStepWaves + wave_row) * R + r;
         if (b >= a.batch) continue;
-        raw_t *orow = reinterpret_cast<raw_t *>(ob + (int64_t)b * a.out_stride_b + c0);
+        raw_t *orow = lane_of(ob + (int64_t)b * a.out_stride_b);
         if (!live[r]) {                               // padding slot: zeros out, state untouched
             *orow = P::zero();
             continue;
         }
-        T *st = sbase + soff[r];
         if (CIRC) {
-            st_state(reinterpret_cast<raw_t *>(st + (int64_t)wpos[r] * a.state_stride_l), xr[r]);
+            st_state(lane_of(st[r]), xr[r]);
         } else {
             // new_state = concat(state, x)[-S:]: rows in front of the window move up by one
             // (reads run ahead of writes), the window rows come straight from registers.
             const int head = S - (W - 1);             // rows in front of the window
-            for (int j = 0; j + 1 < head; ++j)
-                *reinterpret_cast<raw_t *>(st + (int64_t)j * a.state_stride_l) =
-                    *reinterpret_cast<const raw_t *>(st + (int64_t)(j + 1) * a.state_stride_l);
-            if (head > 0) st_state(reinterpret_cast<raw_t *>(st + (int64_t)(head - 1) * a.state_stride_l), rw[r][0]);
+            const int64_t step = a.state_stride_l;
+            T *to = st[r];
+            for (int j = 0; j + 1 < head; ++j, to += step) *lane_of(to) = *lane_of(to + step);
+            if (head > 0) {
+                st_state(lane_of(to), rw[r][0]);
+                to += step;
+            }
 #pragma unroll
-            for (int k = 0; k < W - 2; ++k)
-                st_state(reinterpret_cast<raw_t *>(st + (int64_t)(head + k) * a.state_stride_l), rw[r][k + 1]);
-            st_state(reinterpret_cast<raw_t *>(st + (int64_t)(S - 1) * a.state_stride_l), xr[r]);
+            for (int k = 0; k < W - 2; ++k, to += step) st_state(lane_of(to), rw[r][k + 1]);
+            st_state(lane_of(to), xr[r]);
         }
         float xv[CH], acc[CH], f[W - 1][CH];
 #pragma unroll
@@ -403,21 +439,26 @@ update_tokens_kernel(const TokensArgs ta) {
     Staging staging;
     staging.request(a.weight, a.bias, col0, cols_here);
 
-    const int srow = a.conv_state_indices == nullptr ? b : a.conv_state_indices[b];
-    T *st = reinterpret_cast<T *>(a.conv_state) + (int64_t)(srow < 0 ? 0 : srow) * a.state_stride_b + c0;
-    int cs = 0;
-    if (CIRC) cs = positive_mod(a.cache_seqlens[b], S);
-
+    // As in the step kernel: the x rows wait for nothing, the state rows for the slot and the position.
+    int cs = CIRC ? a.cache_seqlens[b] : 0;
     raw_t rw[W - 1], xr[kMaxTokens];
-#pragma unroll
-    for (int i = 0; i < W - 1; ++i) {
-        const int l = CIRC ? wrap(cs - (W - 1) + i, S) : S - (W - 1) + i;
-        rw[i] = ld_state(reinterpret_cast<const raw_t *>(st + (int64_t)l * a.state_stride_l));
-    }
 #pragma unroll
     for (int i = 0; i < kMaxTokens; ++i) {
         xr[i] = P::zero();
         if (i < L) xr[i] = *reinterpret_cast<const raw_t *>(xrow + (int64_t)i * ta.x_stride_l);
+    }
+    const int srow = a.conv_state_indices == nullptr ? b : a.conv_state_indices[b];
+    T *st = reinterpret_cast<T *>(a.conv_state) + (int64_t)(srow < 0 ? 0 : srow) * a.state_stride_b + c0;
+    int first = S - (W - 1);
+    if (CIRC) {
+        cs = positive_mod(cs, S);
+        first = cs < W - 1 ? cs - (W - 1) + S : cs - (W - 1);
+    }
+    Positions<CIRC> pos(first, a.state_stride_l);
+#pragma unroll
+    for (int i = 0; i < W - 1; ++i) {
+        rw[i] = ld_state(reinterpret_cast<const raw_t *>(st + pos.off));
+        pos.next(a.state_stride_l, S);
     }
 
     staging.publish(staged);
@@ -431,12 +472,11 @@ update_tokens_kernel(const TokensArgs ta) {
     }
 
     if (CIRC) {
-        int wpos = cs;
 #pragma unroll
         for (int i = 0; i < kMaxTokens; ++i) {
             if (i < L) {
-                st_state(reinterpret_cast<raw_t *>(st + (int64_t)wpos * a.state_stride_l), xr[i]);
-                wpos = wpos + 1 == S ? 0 : wpos + 1;
+                st_state(reinterpret_cast<raw_t *>(st + pos.off), xr[i]);
+                pos.next(a.state_stride_l, S);
             }
         }
     } else {
