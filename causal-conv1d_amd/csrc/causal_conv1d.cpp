@@ -145,7 +145,7 @@ void causal_conv1d_fwd(const at::Tensor &x, const at::Tensor &weight,
 }
 
 // overwrite = false: dweight / dbias are added into, as in the reference; true: they are plain
-// outputs and may come in uninitialised.
+// outputs, fp32 or in the type of weight, and may come in uninitialised.
 void bwd_impl(const at::Tensor &x, const at::Tensor &weight,
               const std::optional<at::Tensor> &bias_, at::Tensor &dout,
               const std::optional<at::Tensor> &seq_idx_,
@@ -165,7 +165,8 @@ void bwd_impl(const at::Tensor &x, const at::Tensor &weight,
     CHECK_SHAPE(dweight, dim, width);
     TORCH_CHECK(dout.scalar_type() == x.scalar_type(), "dout must have the dtype of x");
     TORCH_CHECK(dx.scalar_type() == x.scalar_type(), "dx must have the dtype of x");
-    TORCH_CHECK(dweight.scalar_type() == at::ScalarType::Float, "dweight must be float32");
+    const bool in_w_dtype = overwrite && weight.scalar_type() != at::ScalarType::Float && dweight.scalar_type() == weight.scalar_type();
+    TORCH_CHECK(in_w_dtype || dweight.scalar_type() == at::ScalarType::Float, "dweight must be float32");
     check_bias(bias_, weight.scalar_type(), dim);
 
     // dout follows x's layout family; re-lay it out when autograd hands over another one
@@ -181,7 +182,7 @@ void bwd_impl(const at::Tensor &x, const at::Tensor &weight,
     p.x_dtype = to_cc1d_dtype(x.scalar_type(), "x");
     p.w_dtype = to_cc1d_dtype(weight.scalar_type(), "weight");
     p.silu = silu_activation ? 1 : 0;
-    p.overwrite_dweight = overwrite ? 1 : 0;
+    p.overwrite_dweight = in_w_dtype ? CC1D_STORE_IN_W_DTYPE : overwrite ? 1 : 0;
     p.x = x.data_ptr();
     p.x_stride_b = x.stride(0); p.x_stride_c = x.stride(1); p.x_stride_l = x.stride(2);
     p.weight = weight.data_ptr();
@@ -191,14 +192,14 @@ void bwd_impl(const at::Tensor &x, const at::Tensor &weight,
     p.dout_stride_b = dout.stride(0); p.dout_stride_c = dout.stride(1); p.dout_stride_l = dout.stride(2);
     p.dx = dx.data_ptr();
     p.dx_stride_b = dx.stride(0); p.dx_stride_c = dx.stride(1); p.dx_stride_l = dx.stride(2);
-    p.dweight = dweight.data_ptr<float>();
+    p.dweight = static_cast<float *>(dweight.data_ptr());
     p.dw_stride_c = dweight.stride(0); p.dw_stride_w = dweight.stride(1);
     if (dbias_.has_value()) {
         auto &dbias = dbias_.value();
-        TORCH_CHECK(dbias.scalar_type() == at::ScalarType::Float, "dbias must be float32");
+        TORCH_CHECK(dbias.scalar_type() == dweight.scalar_type(), in_w_dtype ? "dbias must have the dtype of dweight" : "dbias must be float32");
         TORCH_CHECK(dbias.is_cuda() && dbias.stride(-1) == 1, "dbias must be a contiguous GPU tensor");
         CHECK_SHAPE(dbias, dim);
-        p.dbias = dbias.data_ptr<float>();
+        p.dbias = static_cast<float *>(dbias.data_ptr());
     }
     if (seq_idx_.has_value()) {
         const auto &seq_idx = seq_idx_.value();
@@ -242,7 +243,24 @@ void bwd_impl(const at::Tensor &x, const at::Tensor &weight,
         workspace = at::empty({(int64_t)ws_bytes}, at::TensorOptions().dtype(at::kByte).device(x.device()));
         ws_ptr = workspace.data_ptr();
     }
-    check_status(cc1d_bwd(&p, ws_ptr, ws_bytes, current_stream()), "causal_conv1d_bwd");
+    const cc1d_stream_t stream = current_stream();
+    const int status = cc1d_bwd(&p, ws_ptr, ws_bytes, stream);
+    if (in_w_dtype && status == CC1D_ERR_TOO_LARGE) {
+        // Launched as slices of the batch that add to one another: the sums in fp32 first.
+        at::Tensor dweight32 = at::empty(dweight.sizes(), dweight.options().dtype(at::kFloat)), dbias32;
+        p.overwrite_dweight = 1;
+        p.dweight = dweight32.data_ptr<float>();
+        p.dw_stride_c = dweight32.stride(0); p.dw_stride_w = dweight32.stride(1);
+        if (dbias_.has_value()) {
+            dbias32 = at::empty(dbias_->sizes(), dweight32.options());
+            p.dbias = dbias32.data_ptr<float>();
+        }
+        check_status(cc1d_bwd(&p, ws_ptr, ws_bytes, stream), "causal_conv1d_bwd");
+        dweight.copy_(dweight32);
+        if (dbias_.has_value()) dbias_->copy_(dbias32);
+        return;
+    }
+    check_status(status, "causal_conv1d_bwd");
 }
 
 void causal_conv1d_bwd(const at::Tensor &x, const at::Tensor &weight,
@@ -423,8 +441,8 @@ void bwd_op(const at::Tensor &x, const at::Tensor &weight, const std::optional<a
                       silu_activation);
 }
 
-// The backward with dweight / dbias as plain outputs (no zero-fill before the call): what the
-// autograd function of this package uses.  Not an op of the reference.
+// The backward with dweight / dbias as plain outputs (no zero-fill before the call), fp32 or in the type of
+// weight: what the autograd function of this package uses.  Not an op of the reference.
 void bwd_overwrite_op(const at::Tensor &x, const at::Tensor &weight, const std::optional<at::Tensor> &bias,
                       const at::Tensor &dout, const std::optional<at::Tensor> &seq_idx,
                       const std::optional<at::Tensor> &initial_states,
@@ -564,8 +582,8 @@ PyObject *forward_call(PyObject *, PyObject *const *a, Py_ssize_t n) {
 }
 
 // (x, weight, bias, dout, seq_idx, initial_states, dfinal_states, return_dinitial_states, silu)
-// -> (dx, dweight, dbias, dinitial_states): every output allocated here, dweight and dbias summed in
-// one fp32 buffer and converted to the parameters' type.
+// -> (dx, dweight, dbias, dinitial_states): every output allocated here, dweight and dbias as one buffer in
+// the parameters' type.
 PyObject *backward_call(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     if (n != 9 || !plain(a[0]) || !plain(a[1]) || !plain_or_none(a[2]) || !plain(a[3]) || !plain_or_none(a[4]) ||
@@ -582,7 +600,8 @@ PyObject *backward_call(PyObject *, PyObject *const *a, Py_ssize_t n) {
         pybind11::gil_scoped_release no_gil;
         const int64_t dim = weight.size(0), width = weight.size(1);
         dx = at::empty_like(x);
-        const at::Tensor sums = at::empty({dim * (width + (bias.has_value() ? 1 : 0))}, x.options().dtype(at::kFloat));
+        const auto type = weight.scalar_type() == at::kHalf || weight.scalar_type() == at::kBFloat16 ? weight.scalar_type() : at::kFloat;
+        const at::Tensor sums = at::empty({dim * (width + (bias.has_value() ? 1 : 0))}, x.options().dtype(type));
         dweight = sums.narrow(0, 0, dim * width).view({dim, width});
         if (bias.has_value()) dbias = sums.narrow(0, dim * width, dim);
         if (return_dinit) dinit = states_like(x, width);

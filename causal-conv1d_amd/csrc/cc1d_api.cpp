@@ -446,6 +446,8 @@ int cc1d_bwd(const cc1d_bwd_params *p, void *workspace, size_t workspace_bytes, 
     }
     if (need > 0 && (workspace == nullptr || !aligned16(workspace) || workspace_bytes < need))
         return CC1D_ERR_WORKSPACE;
+    // Slices add to what the one before them stored, which 16 bits cannot hold.
+    if (p->overwrite_dweight == CC1D_STORE_IN_W_DTYPE && p->w_dtype != CC1D_F32 && !bwd_fits_one_launch(*p)) return CC1D_ERR_TOO_LARGE;
     hipStream_t s = static_cast<hipStream_t>(stream);
     return launch_in_batch_slices(*p, [s, workspace](const cc1d_bwd_params &q) {
         return is_channel_last(q.x_stride_c, q.x_stride_l) ? launch_bwd_channellast(q, workspace, s)

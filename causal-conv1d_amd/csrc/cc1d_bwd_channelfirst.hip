@@ -44,11 +44,6 @@
 namespace cc1d {
 namespace {
 
-// dweight / dbias are added into unless the caller asked for plain stores.
-__device__ __forceinline__ void accumulate(float *dst, float v, int overwrite) {
-    *dst = overwrite ? v : *dst + v;
-}
-
 struct BwdCfGeom {
     int32_t streaming;        // 0: general kernel; streaming kernel with rows 1: on the 16-byte grid, 2: anywhere on it;
                               // 3: short-row kernel (an item is then a group of batch entries, n_segs 1),
@@ -351,8 +346,8 @@ bwd_channelfirst_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float *__res
         if (g.n_parts == 1) {
 #pragma unroll
             for (int w = 0; w < W; ++w)
-                accumulate(p.dweight + (int64_t)c * p.dw_stride_c + (int64_t)w * p.dw_stride_w, dW[w], p.overwrite_dweight);
-            if (p.dbias != nullptr) accumulate(p.dbias + c, dB, p.overwrite_dweight);
+                put_sum(p.dweight, (int64_t)c * p.dw_stride_c + (int64_t)w * p.dw_stride_w, dW[w], sum_store(p));
+            if (p.dbias != nullptr) put_sum(p.dbias, c, dB, sum_store(p));
         } else {
             float *dst = ws + (int64_t)part * (W + 1) * p.dim + c;
 #pragma unroll
@@ -646,8 +641,8 @@ bwd_channelfirst_stream_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float
         if (g.n_parts == 1) {
 #pragma unroll
             for (int w = 0; w < W; ++w)
-                accumulate(p.dweight + (int64_t)c * p.dw_stride_c + (int64_t)w * p.dw_stride_w, dW[w], p.overwrite_dweight);
-            if (p.dbias != nullptr) accumulate(p.dbias + c, dB, p.overwrite_dweight);
+                put_sum(p.dweight, (int64_t)c * p.dw_stride_c + (int64_t)w * p.dw_stride_w, dW[w], sum_store(p));
+            if (p.dbias != nullptr) put_sum(p.dbias, c, dB, sum_store(p));
         } else {
             float *dst = ws + (int64_t)part * (W + 1) * p.dim + c;
 #pragma unroll
@@ -854,8 +849,7 @@ bwd_channelfirst_short_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float 
         if (w < W || (w == W && p.dbias != nullptr)) {
             float total = 0.f;
             for (int i = 0; i < g.n_parts; ++i) total += sums[i][w];
-            accumulate(w < W ? p.dweight + (int64_t)c * p.dw_stride_c + (int64_t)w * p.dw_stride_w : p.dbias + c, total,
-                       p.overwrite_dweight);
+            put_sum(w < W ? p.dweight : p.dbias, w < W ? (int64_t)c * p.dw_stride_c + (int64_t)w * p.dw_stride_w : c, total, sum_store(p));
         }
         return;
     }
@@ -863,8 +857,8 @@ bwd_channelfirst_short_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float 
         if (g.n_parts == 1) {
 #pragma unroll
             for (int w = 0; w < W; ++w)
-                accumulate(p.dweight + (int64_t)c * p.dw_stride_c + (int64_t)w * p.dw_stride_w, dW[w], p.overwrite_dweight);
-            if (p.dbias != nullptr) accumulate(p.dbias + c, dB, p.overwrite_dweight);
+                put_sum(p.dweight, (int64_t)c * p.dw_stride_c + (int64_t)w * p.dw_stride_w, dW[w], sum_store(p));
+            if (p.dbias != nullptr) put_sum(p.dbias, c, dB, sum_store(p));
         } else {
             float *dst = ws + (int64_t)part * (W + 1) * p.dim + c;
 #pragma unroll

@@ -72,7 +72,7 @@ struct BwdCfTileArgs {
     float *ws;                    // [batch * tiles_per_row][W + 1][dim]; unused by DIRECT
     float *dweight, *dbias;       // written by DIRECT
     int64_t dw_stride_c, dw_stride_w;
-    int32_t overwrite;
+    int32_t how;                  // SumStore
     int64_t x_stride_b, x_stride_c, dout_stride_b, dout_stride_c, dx_stride_b, dx_stride_c;   // elements
     int64_t w_stride_c, w_stride_w;
     const void *initial_states;
@@ -381,8 +381,7 @@ bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
         if (w < W || (w == W && a.dbias != nullptr)) {
             float total = 0.f;
             for (int i = 0; i < waves; ++i) total += sums[i * (W + 1) + w];
-            float *dst = w < W ? a.dweight + (int64_t)c * a.dw_stride_c + (int64_t)w * a.dw_stride_w : a.dbias + c;
-            *dst = a.overwrite ? total : *dst + total;
+            put_sum(w < W ? a.dweight : a.dbias, w < W ? (int64_t)c * a.dw_stride_c + (int64_t)w * a.dw_stride_w : c, total, a.how);
         }
         return;
     }
@@ -489,7 +488,7 @@ int launch_bwd_channelfirst_tile(const cc1d_bwd_params &p, float *ws, hipStream_
     a.tiles_per_row = (uint32_t)tiles_per_row(p);
     a.dweight = p.dweight; a.dbias = p.dbias;
     a.dw_stride_c = p.dw_stride_c; a.dw_stride_w = p.dw_stride_w;
-    a.overwrite = p.overwrite_dweight;
+    a.how = sum_store(p);
     a.steps_per_tile = steps_per_tile(p);
     a.total = (uint32_t)((int64_t)p.batch * p.dim * a.tiles_per_row);
     a.seqlen = p.seqlen; a.batch = p.batch; a.dim = p.dim;

@@ -16,7 +16,7 @@ constexpr int kFinChannels = 64;
 __global__ void __launch_bounds__(kFinSlices * kFinChannels)
 bwd_finalize_kernel(const float *__restrict__ ws, int n_parts, int dim, int width,
                     float *__restrict__ dweight, int64_t dw_stride_c, int64_t dw_stride_w,
-                    float *__restrict__ dbias, int overwrite) {
+                    float *__restrict__ dbias, int how) {
     __shared__ float slice_sum[kFinSlices][kFinChannels];
     const int lane = (int)threadIdx.x % kFinChannels;
     const int slice = (int)threadIdx.x / kFinChannels;
@@ -44,8 +44,7 @@ bwd_finalize_kernel(const float *__restrict__ ws, int n_parts, int dim, int widt
         float total = 0.f;
 #pragma unroll
         for (int i = 0; i < kFinSlices; ++i) total += slice_sum[i][lane];
-        float *dst = w < width ? dweight + (int64_t)c * dw_stride_c + (int64_t)w * dw_stride_w : dbias + c;
-        *dst = overwrite ? total : *dst + total;
+        put_sum(w < width ? dweight : dbias, w < width ? (int64_t)c * dw_stride_c + (int64_t)w * dw_stride_w : c, total, how);
     }
 }
 
@@ -54,7 +53,7 @@ int launch_bwd_finalize(const float *ws, int n_parts, const cc1d_bwd_params &p, 
     const uint32_t cblocks = ((uint32_t)p.dim + kFinChannels - 1) / kFinChannels;
     CC1D_LAUNCH(bwd_finalize_kernel, dim3(planes * cblocks), dim3(kFinSlices * kFinChannels), 0, stream,
                        ws, n_parts, p.dim, p.width, p.dweight, p.dw_stride_c, p.dw_stride_w, p.dbias,
-                       p.overwrite_dweight);
+                       sum_store(p));
     return launch_status();
 }
 

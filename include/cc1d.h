@@ -112,7 +112,10 @@ int cc1d_fwd(const cc1d_fwd_params *p, cc1d_stream_t stream);
  * dweight (fp32, (dim, width)) and dbias (fp32, (dim,)) are ACCUMULATED INTO, like the
  * reference (atomicAdd at bwd.cu:243,255 / add_ at causal_conv1d.cpp:452-459): the
  * caller zeroes them first.  With overwrite_dweight = 1 they are plain outputs instead and
- * need no zeroing (two fill launches fewer per backward call).  The reduction always adds
+ * need no zeroing (two fill launches fewer per backward call), and with CC1D_STORE_IN_W_DTYPE plain
+ * outputs in the parameters' own type, each fp32 sum rounded once (to nearest, ties to even) as it is
+ * stored; a problem that needs more than one launch is then refused with CC1D_ERR_TOO_LARGE, since slices
+ * add to one another.  The reduction always adds
  * partial sums in a fixed order, either in a second launch (partials in the workspace) or, for some
  * channel-first launches, in the workgroup that holds all of a channel, so results are
  * bit-reproducible run to run; the reference's `deterministic` switch
@@ -125,12 +128,14 @@ int cc1d_fwd(const cc1d_fwd_params *p, cc1d_stream_t stream);
  * launched as slices of the batch, one after the other on the stream, each adding into
  * dweight / dbias: the sums then follow the slice order (still the same bits run to run).
  * ---------------------------------------------------------------------------------- */
+#define CC1D_STORE_IN_W_DTYPE 2
 typedef struct cc1d_bwd_params {
     int32_t batch, dim, seqlen, width;
     int32_t x_dtype;                 /* of x, dout, dx, initial_states, dfinal_states, dinitial_states */
     int32_t w_dtype;                 /* of weight, bias */
     int32_t silu;
-    int32_t overwrite_dweight;       /* 0: add into dweight / dbias; 1: store the sums, ignore what was there */
+    int32_t overwrite_dweight;       /* 0: add into dweight / dbias; 1: store the sums, ignore what was there;
+                                        CC1D_STORE_IN_W_DTYPE: store them rounded to w_dtype */
 
     const void *x;
     int64_t x_stride_b, x_stride_c, x_stride_l;
@@ -147,7 +152,8 @@ typedef struct cc1d_bwd_params {
 
     void *dx;                        /* same layout family as x */
     int64_t dx_stride_b, dx_stride_c, dx_stride_l;
-    float *dweight;                  /* fp32 (dim, width), accumulated into (or overwritten) */
+    float *dweight;                  /* fp32 (dim, width), accumulated into (or overwritten); elements of
+                                        w_dtype, like dbias, with CC1D_STORE_IN_W_DTYPE */
     int64_t dw_stride_c, dw_stride_w;
     float *dbias;                    /* fp32 (dim,) unit stride, like dweight, or NULL */
     void *dinitial_states;           /* or NULL */
