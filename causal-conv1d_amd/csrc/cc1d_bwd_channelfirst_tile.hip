@@ -57,6 +57,7 @@ typedef void __attribute__((address_space(3))) *lds_ptr_t;
 struct BwdCfTileArgs {
     uint32_t total;               // rows * tiles_per_row wavefronts
     uint32_t tiles_per_row;
+    FastDiv by_tiles, by_inner;   // tiles_per_row; what rows are numbered by (batch or dim)
     int32_t steps_per_tile;       // 64-vector steps of every tile but a row's last, which may have fewer (1 .. 4)
     int32_t seqlen;
     int32_t body_vecs;            // vectors of a row that are walked as vectors (all of them, or a whole number of steps)
@@ -122,8 +123,8 @@ bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
     const int lane = (int)(threadIdx.x & (kWave - 1));
     const uint32_t wid = DIRECT ? (uint32_t)wv : blockIdx.x * (uint32_t)(kBlock / kWave) + (uint32_t)wv;
     if (!DIRECT && wid >= a.total) return;
-    const int tile = (int)(wid % a.tiles_per_row);
-    const uint32_t row = wid / a.tiles_per_row;       // DIRECT: of the channel's rows
+    const uint32_t row = divided(wid, a.by_tiles);    // DIRECT: of the channel's rows
+    const int tile = (int)(wid - row * a.tiles_per_row);
     int b, c;
     if (DIRECT) {
         // XCD x takes workgroups x, x + 8 ..., and its CUs take those in turn: neighbouring channels change
@@ -134,8 +135,11 @@ bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
         b = (int)row;
         c = (int)(other < (uint32_t)a.dim ? other : blockIdx.x);
     }
-    else if (a.batch_inner) { b = (int)(row % (uint32_t)a.batch); c = (int)(row / (uint32_t)a.batch); }
-    else { c = (int)(row % (uint32_t)a.dim); b = (int)(row / (uint32_t)a.dim); }
+    else {
+        const uint32_t outer = divided(row, a.by_inner), inner = row - outer * (uint32_t)(a.batch_inner ? a.batch : a.dim);
+        b = (int)(a.batch_inner ? inner : outer);
+        c = (int)(a.batch_inner ? outer : inner);
+    }
     const int L = a.seqlen;
 
     const T *xrow = reinterpret_cast<const T *>(a.x) + (int64_t)b * a.x_stride_b + (int64_t)c * a.x_stride_c;
@@ -495,6 +499,8 @@ int launch_bwd_channelfirst_tile(const cc1d_bwd_params &p, float *ws, hipStream_
     a.tail_vecs = tail_vecs_of_row(p);
     a.body_vecs = (int32_t)(((int64_t)p.seqlen + vec_elems(p.x_dtype) - 1) / vec_elems(p.x_dtype)) - a.tail_vecs;
     a.batch_inner = p.batch > 1 && p.dim > 1 && p.x_stride_b < p.x_stride_c ? 1 : 0;
+    a.by_tiles = fast_div(a.tiles_per_row);
+    a.by_inner = fast_div((uint32_t)(a.batch_inner ? p.batch : p.dim));
     a.w_dtype = p.w_dtype;
     a.x = p.x; a.dout = p.dout; a.dx = p.dx; a.weight = p.weight; a.bias = p.bias; a.ws = ws;
     a.x_stride_b = p.x_stride_b; a.x_stride_c = p.x_stride_c;

@@ -138,6 +138,9 @@ bool make_geom(const cc1d_bwd_params &p, BwdClGeom &g) {
     if (g.blocks_per_chunk != 0)
         g.blocks_per_xcd = (g.blocks_per_xcd + g.blocks_per_chunk - 1) / g.blocks_per_chunk * g.blocks_per_chunk;
     if ((int64_t)g.blocks_per_xcd * kXcds * kBlock >= thread_limit()) return false;
+    g.by_chunk = fast_div(g.blocks_per_chunk);
+    g.by_row = fast_div(g.waves_per_row);
+    g.by_quads = fast_div((uint32_t)g.n_quads);
     g.w_mode = weights_mode(p.weight, p.bias, p.w_dtype, p.x_dtype, p.w_stride_c, p.w_stride_w, p.width);
     return true;
 }

@@ -61,6 +61,7 @@ struct BwdClGeom {
     uint32_t total;           // batch * n_quads * waves_per_row workgroups
     uint32_t blocks_per_xcd;  // grid size / 8
     uint32_t blocks_per_chunk; // workgroups an XCD takes in a row before the next XCD's (0: its whole slice)
+    FastDiv by_chunk, by_row, by_quads;   // blocks_per_chunk, waves_per_row, n_quads
     int32_t w_mode;           // weights_mode: 0 general loader, 1 / 2 packed taps
     int32_t channels_per_lane;
 };
@@ -477,18 +478,18 @@ bwd_channellast_kernel(const cc1d_bwd_params p, const BwdClGeom g, float *__rest
     // XCD x executes workgroups x, x+8, x+16, ...; give it chunks of consecutive runs, the 8 XCDs
     // side by side on 8 neighbouring chunks (or, blocks_per_chunk == 0, the x-th contiguous slice).
     const uint32_t xcd = blockIdx.x % kXcds, nth = blockIdx.x / kXcds;
-    const uint32_t block = g.blocks_per_chunk == 0
-                               ? xcd * g.blocks_per_xcd + nth
-                               : ((nth / g.blocks_per_chunk) * kXcds + xcd) * g.blocks_per_chunk + nth % g.blocks_per_chunk;
+    const uint32_t chunk = divided(nth, g.by_chunk);
+    const uint32_t block = g.blocks_per_chunk == 0 ? xcd * g.blocks_per_xcd + nth
+                                                   : nth + (chunk * (uint32_t)(kXcds - 1) + xcd) * g.blocks_per_chunk;
     // A workgroup takes 64 adjacent vector-columns of four consecutive runs of one sequence,
     // one run per wavefront: a wavefront's row range and the sub-sequence ids it reads are
     // scalars.  Neighbouring workgroups take neighbouring columns of the same rows.
     const int wv_in_block = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const int lane = (int)(threadIdx.x & (kWave - 1));
-    const uint32_t col = (block % g.waves_per_row) * (uint32_t)kWave + (uint32_t)lane;
-    const uint32_t bq = block / g.waves_per_row;
-    const int quad = (int)(bq % (uint32_t)g.n_quads);
-    const int b = (int)(bq / (uint32_t)g.n_quads);
+    const uint32_t bq = divided(block, g.by_row);
+    const uint32_t col = (block - bq * g.waves_per_row) * (uint32_t)kWave + (uint32_t)lane;
+    const int b = (int)divided(bq, g.by_quads);
+    const int quad = (int)bq - b * g.n_quads;
     const int run = quad * kRunsPerBlock + wv_in_block;
 
     float dW[CH][W], dB[CH];

@@ -21,6 +21,17 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 constexpr int kWave = 64;
 constexpr int kBlock = 256;  // 4 wavefronts per workgroup
 
+// A divisor as a factor of the quotient's upper word (device.hpp: divided).  For 2^l < d <= 2^(l+1) the factor is
+// 2^(32+l) / d rounded up: below 2^32, and off by less than d / 2^(32+l), so exact for every n < 2^31.
+struct FastDiv {
+    uint32_t mul, shift;                              // mul 0: a division by one
+};
+inline FastDiv fast_div(uint32_t d) {
+    if (d <= 1) return {0, 0};
+    const uint32_t l = 31 - (uint32_t)__builtin_clz(d - 1);
+    return {(uint32_t)((((uint64_t)1 << (32 + l)) + d - 1) / d), l};
+}
+
 template <typename To, typename From>
 __device__ __forceinline__ To bitcast(const From &v) {
     return __builtin_bit_cast(To, v);
@@ -450,6 +461,12 @@ __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, kWave);
     return v;
+}
+
+// n / d for a d that the host knows (fast_div): two scalar instructions for wave-uniform numbers instead of
+// two dozen with a reciprocal among them, in front of a wavefront's first request.  n < 2^31.
+__device__ __forceinline__ uint32_t divided(uint32_t n, const FastDiv &d) {
+    return d.mul == 0 ? n : __umulhi(n, d.mul) >> d.shift;
 }
 
 // ---------------------------------------------------------------------------------

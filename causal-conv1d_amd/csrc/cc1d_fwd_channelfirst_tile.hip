@@ -43,6 +43,7 @@ typedef void __attribute__((address_space(3))) *lds_ptr_t;
 struct FwdCfTileArgs {
     uint32_t total;               // rows * tiles_per_row wavefronts
     uint32_t tiles_per_row;
+    FastDiv by_tiles, by_inner;   // tiles_per_row; what rows are numbered by (batch or dim)
     int32_t seqlen;
     int32_t body_vecs;            // vectors of a row that are walked as vectors (all of them, or a whole number of steps)
     int32_t tail_vecs;            // vectors behind them, done one position per lane (0: none)
@@ -77,14 +78,13 @@ fwd_channelfirst_tile_kernel(const FwdCfTileArgs a) {
     const int lane = (int)(threadIdx.x & (kWave - 1));
     const uint32_t wid = blockIdx.x * (uint32_t)(kBlock / kWave) + (uint32_t)wv;
     if (wid >= a.total) return;
-    const int tile = (int)(wid % a.tiles_per_row);
-    const uint32_t row = wid / a.tiles_per_row;
+    const uint32_t row = divided(wid, a.by_tiles);
+    const int tile = (int)(wid - row * a.tiles_per_row);
     // Channels run fastest for tensors whose rows lie in (batch, dim) order in memory; for a
     // (dim, batch, seqlen) tensor seen as (batch, dim, seqlen) the batch entries of a channel are
     // the neighbours in memory and run fastest instead.
-    int b, c;
-    if (a.batch_inner) { b = (int)(row % (uint32_t)a.batch); c = (int)(row / (uint32_t)a.batch); }
-    else { c = (int)(row % (uint32_t)a.dim); b = (int)(row / (uint32_t)a.dim); }
+    const uint32_t outer = divided(row, a.by_inner), inner = row - outer * (uint32_t)(a.batch_inner ? a.batch : a.dim);
+    const int b = (int)(a.batch_inner ? inner : outer), c = (int)(a.batch_inner ? outer : inner);
 
     const T *xrow = reinterpret_cast<const T *>(a.x) + (int64_t)b * a.x_stride_b + (int64_t)c * a.x_stride_c;
     T *orow = reinterpret_cast<T *>(a.out) + (int64_t)b * a.out_stride_b + (int64_t)c * a.out_stride_c;
@@ -278,6 +278,8 @@ int launch_fwd_channelfirst_tile(const cc1d_fwd_params &p, hipStream_t stream) {
     a.total = (uint32_t)total;
     a.batch = p.batch; a.dim = p.dim;
     a.batch_inner = p.batch > 1 && p.dim > 1 && p.x_stride_b < p.x_stride_c ? 1 : 0;
+    a.by_tiles = fast_div(a.tiles_per_row);
+    a.by_inner = fast_div((uint32_t)(a.batch_inner ? p.batch : p.dim));
     a.w_dtype = p.w_dtype;
     a.states = (p.initial_states != nullptr ? 1 : 0) | (p.final_states != nullptr ? 2 : 0);
     a.x = p.x; a.out = p.out; a.weight = p.weight; a.bias = p.bias;

@@ -59,6 +59,7 @@ typedef void __attribute__((address_space(3))) *lds_ptr_t;
 struct FwdClArgs {
     uint32_t blocks_per_xcd;   // grid size / 8
     uint32_t blocks_per_chunk; // workgroups an XCD takes in a row before the next XCD's (0: its whole slice)
+    FastDiv by_chunk, by_row, by_runs;   // blocks_per_chunk, waves_per_row, n_runs
     uint32_t first_tail_block; // workgroups from here on run the varlen gather
     uint32_t total;            // batch * n_runs * waves_per_row wavefronts
     uint32_t waves_per_row;    // ceil(n_cols / 64): wavefronts side by side on one row
@@ -111,19 +112,19 @@ fwd_channellast_kernel(const FwdClArgs a, const FwdClRare q) {
     }
     // XCD x executes workgroups x, x+8, x+16, ...
     const uint32_t xcd = blockIdx.x % kXcds, nth = blockIdx.x / kXcds;
-    const uint32_t block = a.blocks_per_chunk == 0
-                               ? xcd * a.blocks_per_xcd + nth
-                               : ((nth / a.blocks_per_chunk) * kXcds + xcd) * a.blocks_per_chunk + nth % a.blocks_per_chunk;
+    const uint32_t chunk = divided(nth, a.by_chunk);
+    const uint32_t block = a.blocks_per_chunk == 0 ? xcd * a.blocks_per_xcd + nth
+                                                   : nth + (chunk * (uint32_t)(kXcds - 1) + xcd) * a.blocks_per_chunk;
     // A wavefront never straddles two runs: its batch index, run and row range are scalars,
     // and so are the sub-sequence ids it reads.
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const int lane = (int)(threadIdx.x & (kWave - 1));
     const uint32_t wave = block * (uint32_t)(kBlock / kWave) + (uint32_t)wv;
     if (wave >= a.total) return;
-    const uint32_t col = (wave % a.waves_per_row) * (uint32_t)kWave + (uint32_t)lane;
-    const uint32_t rb = wave / a.waves_per_row;
-    const int run = (int)(rb % (uint32_t)a.n_runs);
-    const int b = (int)(rb / (uint32_t)a.n_runs);
+    const uint32_t rb = divided(wave, a.by_row);
+    const uint32_t col = (wave - rb * a.waves_per_row) * (uint32_t)kWave + (uint32_t)lane;
+    const int b = (int)divided(rb, a.by_runs);
+    const int run = (int)rb - b * a.n_runs;
     const int L = a.seqlen;
     const bool has_init = (a.states & 1) != 0;
     const int T = TS != 0 ? TS : a.rows_per_run;
@@ -436,6 +437,9 @@ int launch_fwd_channellast(const cc1d_fwd_params &p, const cc1d_varlen_params *g
     if (a.blocks_per_chunk != 0)
         a.blocks_per_xcd = (a.blocks_per_xcd + a.blocks_per_chunk - 1) / a.blocks_per_chunk * a.blocks_per_chunk;
     if ((int64_t)a.blocks_per_xcd * kXcds * kBlock >= thread_limit()) return CC1D_ERR_TOO_LARGE;
+    a.by_chunk = fast_div(a.blocks_per_chunk);
+    a.by_row = fast_div(a.waves_per_row);
+    a.by_runs = fast_div((uint32_t)a.n_runs);
     a.first_tail_block = a.blocks_per_xcd * kXcds;
     a.seqlen = p.seqlen;
     a.x_row_bytes = (uint32_t)(p.x_stride_l * eb);
