@@ -833,38 +833,26 @@ bwd_channelfirst_short_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float 
         }
     }
 
-    // One fixed-order reduction over the wave, then a single writer.
-#pragma unroll
-    for (int w = 0; w < W; ++w) dW[w] = wave_sum(dW[w]);
-    dB = wave_sum(dB);
+    // One fixed-order reduction over the wave; the lane that holds a sum moves it.
+    const float sum = wave_sums<W>(dW, dB, lane);
+    const int which = lane < W ? lane : lane == 4 ? W : -1;
+    auto hand_over = [&](int w, float total) __attribute__((always_inline)) {
+        put_sum(w < W ? p.dweight : p.dbias, w < W ? (int64_t)c * p.dw_stride_c + (int64_t)w * p.dw_stride_w : c, total, sum_store(p));
+    };
     if constexpr (DIRECT) {
         __shared__ float sums[kMaxDirectParts][W + 1];
-        if (lane == 0) {
-#pragma unroll
-            for (int w = 0; w < W; ++w) sums[part][w] = dW[w];
-            sums[part][W] = dB;
-        }
+        if (which >= 0) sums[part][which] = sum;
         __syncthreads();
         const int w = (int)threadIdx.x;
         if (w < W || (w == W && p.dbias != nullptr)) {
             float total = 0.f;
             for (int i = 0; i < g.n_parts; ++i) total += sums[i][w];
-            put_sum(w < W ? p.dweight : p.dbias, w < W ? (int64_t)c * p.dw_stride_c + (int64_t)w * p.dw_stride_w : c, total, sum_store(p));
+            hand_over(w, total);
         }
-        return;
-    }
-    if (lane == 0) {
-        if (g.n_parts == 1) {
-#pragma unroll
-            for (int w = 0; w < W; ++w)
-                put_sum(p.dweight, (int64_t)c * p.dw_stride_c + (int64_t)w * p.dw_stride_w, dW[w], sum_store(p));
-            if (p.dbias != nullptr) put_sum(p.dbias, c, dB, sum_store(p));
-        } else {
-            float *dst = ws + (int64_t)part * (W + 1) * p.dim + c;
-#pragma unroll
-            for (int w = 0; w < W; ++w) dst[(int64_t)w * p.dim] = dW[w];
-            dst[(int64_t)W * p.dim] = dB;
-        }
+    } else if (g.n_parts == 1) {
+        if (which >= 0 && (which < W || p.dbias != nullptr)) hand_over(which, sum);
+    } else if (which >= 0) {
+        ws[((int64_t)part * (W + 1) + which) * p.dim + c] = sum;
     }
 }
 

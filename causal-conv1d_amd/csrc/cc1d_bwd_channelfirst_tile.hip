@@ -84,18 +84,6 @@ struct BwdCfTileArgs {
     int64_t dinit_stride_b, dinit_stride_c, dinit_stride_l;
 };
 
-// Sum over the 64 lanes in a fixed order, result in lane 63: prefix sums inside each row of 16
-// lanes (row_shr 1, 2, 4, 8), then the rows' totals across (row_bcast 15, 31).
-__device__ __forceinline__ float wave_total_in_lane63(float v) {
-    v += bitcast<float>(__builtin_amdgcn_update_dpp(0, bitcast<int>(v), 0x111, 0xf, 0xf, true));
-    v += bitcast<float>(__builtin_amdgcn_update_dpp(0, bitcast<int>(v), 0x112, 0xf, 0xf, true));
-    v += bitcast<float>(__builtin_amdgcn_update_dpp(0, bitcast<int>(v), 0x114, 0xf, 0xf, true));
-    v += bitcast<float>(__builtin_amdgcn_update_dpp(0, bitcast<int>(v), 0x118, 0xf, 0xf, true));
-    v += bitcast<float>(__builtin_amdgcn_update_dpp(0, bitcast<int>(v), 0x142, 0xa, 0xf, true));   // row_bcast:15 into rows 1, 3
-    v += bitcast<float>(__builtin_amdgcn_update_dpp(0, bitcast<int>(v), 0x143, 0xc, 0xf, true));   // row_bcast:31 into rows 2, 3
-    return v;
-}
-
 // DIRECT: a workgroup is one channel and its wavefronts are the channel's tiles, so that it can add up
 // their sums itself and store dweight / dbias: one launch instead of two, and no workspace
 // traffic.  Otherwise the wavefronts are numbered along the rows, four to a workgroup, and leave their
@@ -365,21 +353,17 @@ bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
         }
     }
 
-    // The tile's sums over its lanes, in a fixed order, to plane (batch entry, tile) of the workspace.
-#pragma unroll
-    for (int w = 0; w < W; ++w) dW[w] = wave_total_in_lane63(dW[w]);
-    dB = wave_total_in_lane63(dB);
+    // The tile's sums over its lanes, in a fixed order, to plane (batch entry, tile) of the workspace: the
+    // lane that holds one moves it.
+    const float sum = wave_sums<W>(dW, dB, lane);
+    const int which = lane < W ? lane : lane == 4 ? W : -1;
     if constexpr (DIRECT) {
         // The channel's tiles are this workgroup's wavefronts: their sums are added in order and stored.
         // (not blockDim: a kernel that asks for its launch shape takes 256 bytes of hidden arguments, and
         // every byte of a launch's arguments costs about 3 ns of host time)
         const int waves = a.batch * (int)a.tiles_per_row;
         float *sums = reinterpret_cast<float *>(lds + waves * XV);
-        if (lane == kWave - 1) {
-#pragma unroll
-            for (int w = 0; w < W; ++w) sums[wv * (W + 1) + w] = dW[w];
-            sums[wv * (W + 1) + W] = dB;
-        }
+        if (which >= 0) sums[wv * (W + 1) + which] = sum;
         __syncthreads();
         const int w = (int)threadIdx.x;
         if (w < W || (w == W && a.dbias != nullptr)) {
@@ -389,12 +373,7 @@ bwd_channelfirst_tile_kernel(const BwdCfTileArgs a) {
         }
         return;
     }
-    if (lane == kWave - 1) {
-        float *dst = a.ws + ((int64_t)b * a.tiles_per_row + tile) * (int64_t)(W + 1) * a.dim + c;
-#pragma unroll
-        for (int w = 0; w < W; ++w) dst[(int64_t)w * a.dim] = dW[w];
-        dst[(int64_t)W * a.dim] = dB;
-    }
+    if (which >= 0) a.ws[(((int64_t)b * a.tiles_per_row + tile) * (W + 1) + which) * a.dim + c] = sum;
 }
 
 // LDS of one wavefront: steps_per_tile steps of x, the vectors around them, room for a tail, its sums.
