@@ -47,13 +47,14 @@ namespace {
 struct BwdCfGeom {
     int32_t streaming;        // 0: general kernel; streaming kernel with rows 1: on the 16-byte grid, 2: anywhere on it;
                               // 3: short-row kernel (an item is then a group of batch entries, n_segs 1),
-                              // 4: the same with element accesses
+                              // 4: the same for rows anywhere in memory
     int32_t vecs_per_seg;     // multiple of 64
     int32_t n_segs;           // segments per row
     int32_t n_items;          // batch * n_segs
     int32_t n_parts;          // slices of the item list per channel
     int32_t items_per_part;
     int32_t lanes_log2;       // short-row kernel (streaming 3, 4): log2 of the lanes one row takes
+    FastDiv by_parts;         // n_parts, for the short rows
 };
 
 template <int DT>
@@ -660,35 +661,63 @@ constexpr int kMaxDirectParts = 16;
 // previous lane (vector 0: zeros or initial_states), g's from the next lane (last vector: zeros),
 // and an item is one load of x, one of dout and one store of dx per lane.  Formulas, operation
 // order and the reduction at the end are those of the kernels above.
-// ALIGNED: rows of whole vectors, every tensor on one 16-byte grid.  ALIGNED = false: rows of any
-// length (down to 1) anywhere in memory, the same lanes, with a lane's up to VEC positions read
-// and written element by element (positions past the row's end read as zero).
+// ROWS: kWhole, rows of whole vectors, every tensor on one 16-byte grid; kAnywhere, rows of a vector and more
+// anywhere in memory: the lane of a row's last, partly filled vector reads the row's last 16 bytes instead, drops
+// what the lane in front of it owns, and stores its part in pieces of 8, 4 and 2 bytes (storing the row's last
+// 16 bytes too, the shared ones with the same values as the lane in front, took (4, 1024, 300) bf16 from 8 us to
+// 22: overlapping stores of a wavefront are slow); kElements, rows shorter than a vector, read and written
+// element by element, as all rows off the grid were.  Positions past the row's end count as zero.
 // DIRECT: the parts of a channel, two to sixteen, are the wavefronts of one workgroup, which adds up
 // their sums and stores dweight / dbias itself.  The wavefronts take the same rows in the same order as
 // without it; what goes is the second launch, 2-5 us behind a kernel that may run for less (see
 // short_rows_direct for where that is worth it).
-template <int DT, int W, bool ALIGNED, bool DIRECT>
+enum ShortRows : int { kWhole, kAnywhere, kElements };
+template <int DT, int W, int ROWS, bool DIRECT>
 __global__ void __launch_bounds__(DIRECT ? kMaxDirectParts * kWave : kBlock)
 bwd_channelfirst_short_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float *__restrict__ ws) {
     using E = Elem<DT>;
     constexpr int VEC = E::kVec;
     constexpr bool PRECISE = E::kPreciseAct;
 
-    const uint32_t wid = DIRECT ? blockIdx.x * (uint32_t)g.n_parts + threadIdx.x / kWave
-                                : (blockIdx.x * (uint32_t)kBlock + threadIdx.x) / kWave;
+    // Off the grid the channel is a scalar and the first item's rows are asked for in front of the taps:
+    // accesses of any address and the shifts leave fewer registers.  Otherwise the wavefront's number stays
+    // in a vector register and the rows follow the taps, (16, 512, 256) bf16 5.4 us against 5.9.
+    constexpr bool EARLY = ROWS == kAnywhere;
+    const uint32_t wv_in_block = EARLY ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave)) : threadIdx.x / kWave;
+    const uint32_t wid = blockIdx.x * (DIRECT ? (uint32_t)g.n_parts : (uint32_t)(kBlock / kWave)) + wv_in_block;
     const int lane = threadIdx.x & (kWave - 1);
     if (!DIRECT && wid >= (uint32_t)p.dim * (uint32_t)g.n_parts) return;     // whole wave leaves together
-    const int part = (int)(wid % (uint32_t)g.n_parts);
-    const int c = (int)(wid / (uint32_t)g.n_parts);
+    const int c = EARLY && DIRECT ? (int)blockIdx.x : (int)divided(wid, g.by_parts);
+    const int part = (int)(wid - (uint32_t)c * (uint32_t)g.n_parts);
     const int L = p.seqlen;
     const int n_vecs = (L + VEC - 1) / VEC;
     const int v = lane & ((1 << g.lanes_log2) - 1);
     const int r = lane >> g.lanes_log2;
     const int rows_per_item = kWave >> g.lanes_log2;
     const bool silu_on = p.silu != 0;
+    // kAnywhere: how many bytes of the row's last 16 the lane of its last vector shares with the lane in front of it.
+    const int shared = ROWS == kAnywhere && v == n_vecs - 1 ? (n_vecs * VEC - L) * E::kBytes : 0;
+    const int first = v * VEC - shared / E::kBytes;   // the lane's first position in memory
+
+    const int item_begin = part * g.items_per_part;
+    int item_end = item_begin + g.items_per_part;
+    if (item_end > g.n_items) item_end = g.n_items;
+
+    u32x4 rx = u32x4{0u, 0u, 0u, 0u}, rd = u32x4{0u, 0u, 0u, 0u};
+    auto fetch = [&](int item) __attribute__((always_inline)) {
+        const int b_here = item * rows_per_item + r;
+        if (ROWS != kElements && b_here < p.batch && v < n_vecs) {
+            const int64_t xrow = (int64_t)b_here * p.x_stride_b + (int64_t)c * p.x_stride_c;
+            const int64_t drow = (int64_t)b_here * p.dout_stride_b + (int64_t)c * p.dout_stride_c;
+            rx = ROWS == kWhole ? ld_vec_nt<DT>(p.x, xrow + first) : ld_vec_any<DT>(p.x, xrow + first);
+            rd = ROWS == kWhole ? ld_vec_nt<DT>(p.dout, drow + first) : ld_vec_any<DT>(p.dout, drow + first);
+        }
+    };
+    if (EARLY) fetch(item_begin);
 
     float wv[W], bias_v;
-    channel_taps<W>(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, c, wv, bias_v);
+    if (EARLY) uniform_taps<W>(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, c, wv, bias_v);
+    else channel_taps<W>(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, c, wv, bias_v);
     float wvs[W];
 #pragma unroll
     for (int w = 0; w < W; ++w) wvs[w] = wv[w] * kSiluPrescale;
@@ -698,11 +727,8 @@ bwd_channelfirst_short_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float 
 #pragma unroll
     for (int w = 0; w < W; ++w) dW[w] = 0.f;
 
-    const int item_begin = part * g.items_per_part;
-    int item_end = item_begin + g.items_per_part;
-    if (item_end > g.n_items) item_end = g.n_items;
-
     for (int item = item_begin; item < item_end; ++item) {
+        if (!EARLY) fetch(item);
         // Lanes without a vector of their own stay in step (the lane shifts need every lane) on
         // entry 0's addresses; they load zeros, add zeros to the sums and store nothing.
         const int b_here = item * rows_per_item + r;
@@ -713,14 +739,10 @@ bwd_channelfirst_short_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float 
         const int64_t dxrow = (int64_t)b * p.dx_stride_b + (int64_t)c * p.dx_stride_c;
 
         float xf[VEC], gf[VEC];
-        if (ALIGNED) {
-            u32x4 rx = u32x4{0u, 0u, 0u, 0u}, rd = u32x4{0u, 0u, 0u, 0u};
-            if (mine) {
-                rx = ld_vec_nt<DT>(p.x, xrow + (int64_t)v * VEC);
-                rd = ld_vec_nt<DT>(p.dout, drow + (int64_t)v * VEC);
-            }
-            E::unpack(rx, xf);
-            E::unpack(rd, gf);
+        if (ROWS != kElements) {
+            if (!mine) rx = rd = u32x4{0u, 0u, 0u, 0u};
+            E::unpack(ROWS == kAnywhere ? without_front(rx, shared) : rx, xf);
+            E::unpack(ROWS == kAnywhere ? without_front(rd, shared) : rd, gf);
         } else {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) xf[e] = gf[e] = 0.f;
@@ -780,7 +802,7 @@ bwd_channelfirst_short_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float 
             dxv[e] = a;
         }
         // The row's last W-1 positions take dfinal_states (whole vectors: all in the last one).
-        if (ALIGNED) {
+        if (ROWS == kWhole) {
             if (p.dfinal_states != nullptr && mine && v == n_vecs - 1) {
 #pragma unroll
                 for (int i = 0; i < W - 1; ++i)
@@ -788,21 +810,25 @@ bwd_channelfirst_short_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float 
                                                                                (int64_t)c * p.dfinal_stride_c +
                                                                                (int64_t)i * p.dfinal_stride_l);
             }
-            if (mine) st_vec_nt<DT>(p.dx, dxrow + (int64_t)v * VEC, E::pack(dxv));
-        } else if (mine) {
-            if (p.dfinal_states != nullptr && (v + 1) * VEC > L - (W - 1)) {
+            if (mine) st_vec_nt<DT>(p.dx, dxrow + first, E::pack(dxv));
+        } else {
+            if (p.dfinal_states != nullptr && mine && (v + 1) * VEC > L - (W - 1)) {
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) {
-                    const int t = v * VEC + e;
-                    if (t >= L - (W - 1) && t < L)
-                        dxv[e] += ld_elem<DT>(p.dfinal_states, (int64_t)b * p.dfinal_stride_b +
-                                                                   (int64_t)c * p.dfinal_stride_c +
-                                                                   (int64_t)(t - (L - (W - 1))) * p.dfinal_stride_l);
+                for (int i = 0; i < W - 1; ++i) {
+                    const int at = L - (W - 1) + i - v * VEC;      // the position's place in the lane's vector, or outside of it
+                    const float d = ld_elem<DT>(p.dfinal_states, (int64_t)b * p.dfinal_stride_b + (int64_t)c * p.dfinal_stride_c +
+                                                                     (int64_t)i * p.dfinal_stride_l);
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) dxv[e] = at == e ? dxv[e] + d : dxv[e];
                 }
             }
+            if (ROWS == kAnywhere) {
+                if (mine) st_front_any<DT>(p.dx, dxrow + v * VEC, E::pack(dxv), shared == 0, VEC - (n_vecs * VEC - L));
+            } else if (mine) {
 #pragma unroll
-            for (int e = 0; e < VEC; ++e)
-                if (v * VEC + e < L) st_elem<DT>(p.dx, dxrow + v * VEC + e, dxv[e]);
+                for (int e = 0; e < VEC; ++e)
+                    if (v * VEC + e < L) st_elem<DT>(p.dx, dxrow + v * VEC + e, dxv[e]);
+            }
         }
 
 #pragma unroll
@@ -824,13 +850,14 @@ bwd_channelfirst_short_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float 
                     const int t = i - (W - 1) + k;
                     a = fmaf(wv[W - 1 - k], t >= 0 ? gf[t] : 0.f, a);
                 }
-                if (!ALIGNED && p.dfinal_states != nullptr && i >= L)
+                if (ROWS == kElements && p.dfinal_states != nullptr && i >= L)
                     a += ld_elem<DT>(p.dfinal_states, (int64_t)b * p.dfinal_stride_b + (int64_t)c * p.dfinal_stride_c +
                                                           (int64_t)(i - L) * p.dfinal_stride_l);
                 st_elem<DT>(p.dinitial_states, (int64_t)b * p.dinit_stride_b + (int64_t)c * p.dinit_stride_c +
                                                    (int64_t)i * p.dinit_stride_l, a);
             }
         }
+        if (EARLY && item + 1 < item_end) fetch(item + 1);
     }
 
     // One fixed-order reduction over the wave; the lane that holds a sum moves it.
@@ -879,14 +906,16 @@ BwdCfGeom make_geom(const cc1d_bwd_params &p) {
     const int64_t max_parts = (int64_t)p.batch * max_steps;
     if (parts > max_parts) parts = max_parts;
     if (parts < 1) parts = 1;
-    BwdCfGeom g;
+    BwdCfGeom g = {};
     const bool on_grid = aligned16(p.x) && p.x_stride_b % vec == 0 && p.x_stride_c % vec == 0 && p.seqlen % vec == 0;
     g.lanes_log2 = 0;
     // Short rows of whole vectors with every tensor on one grid: several batch entries to a
     // wavefront, an item is a group of them.  (16, 5376, 128) bf16 57.2 -> 16.0 us, fp32 43.0 -> 25.0 us;
     // (4, 5376, 256) bf16 18.2 -> 10.3 us.
-    // Rows that are not whole vectors on one grid take the same lanes with element accesses:
-    // (16, 5376, 100) bf16 107 -> 39 us, (64, 2048, 60) 165 -> 36 us, (256, 5376, 4) 1514 -> 73 us.
+    // Rows that are not whole vectors on one grid take the same lanes, vectors of any address and the last one of
+    // a row in pieces; rows shorter than a vector take single elements.  Against elements throughout:
+    // (8, 4096, 500) bf16 59.8 -> 25.6 us, (16, 2048, 511) 65.9 -> 29.6, (32, 1024, 99) fp16 19.3 -> 11.2, (1, 4096, 333) bf16
+    // 8.7 -> 6.3, (8, 2048, 250) fp32 22.1 -> 15.4; (256, 5376, 4) 1514 -> 73 us walking -> elements.
     const int64_t n_vecs = ((int64_t)p.seqlen + vec - 1) / vec;
     if (n_vecs <= kWave) {
         const bool aligned = on_grid &&
@@ -901,6 +930,7 @@ BwdCfGeom make_geom(const cc1d_bwd_params &p) {
         if (parts > g.n_items) parts = g.n_items;
         g.items_per_part = (int32_t)((g.n_items + parts - 1) / parts);
         g.n_parts = (g.n_items + g.items_per_part - 1) / g.items_per_part;
+        g.by_parts = fast_div((uint32_t)g.n_parts);
         return g;
     }
     // The chip holds about 4096 of these wavefronts at once.  A launch of 1 to 1.5 times that many
@@ -959,15 +989,15 @@ bool short_rows_direct(const cc1d_bwd_params &p, const BwdCfGeom &g) {
     return g.n_parts <= most_parts && g.items_per_part <= most_items;
 }
 
-template <int DT, bool ALIGNED>
+template <int DT, int ROWS>
 int launch_short(const cc1d_bwd_params &p, const BwdCfGeom &g, float *ws, hipStream_t stream) {
     const bool direct = short_rows_direct(p, g);
     const uint32_t waves = direct ? (uint32_t)g.n_parts : (uint32_t)(kBlock / kWave);
     const uint32_t blocks = (uint32_t)(((int64_t)p.dim * g.n_parts + waves - 1) / waves);
     auto launch = [&](auto width) {
         constexpr int W = decltype(width)::value;
-        if (direct) CC1D_LAUNCH((bwd_channelfirst_short_kernel<DT, W, ALIGNED, true>), dim3(blocks), dim3(waves * kWave), 0, stream, p, g, ws);
-        else CC1D_LAUNCH((bwd_channelfirst_short_kernel<DT, W, ALIGNED, false>), dim3(blocks), dim3(waves * kWave), 0, stream, p, g, ws);
+        if (direct) CC1D_LAUNCH((bwd_channelfirst_short_kernel<DT, W, ROWS, true>), dim3(blocks), dim3(waves * kWave), 0, stream, p, g, ws);
+        else CC1D_LAUNCH((bwd_channelfirst_short_kernel<DT, W, ROWS, false>), dim3(blocks), dim3(waves * kWave), 0, stream, p, g, ws);
     };
     switch (p.width) {
         case 2: launch(std::integral_constant<int, 2>{}); break;
@@ -982,8 +1012,9 @@ int launch_dtype(const cc1d_bwd_params &p, const BwdCfGeom &g, float *ws, hipStr
     const int64_t waves = (int64_t)p.dim * g.n_parts;
     if (waves >= wave_limit()) return CC1D_ERR_TOO_LARGE;
     const uint32_t blocks = (uint32_t)((waves + (kBlock / kWave) - 1) / (kBlock / kWave));
-    if (g.streaming == 3) return launch_short<DT, true>(p, g, ws, stream);    // short rows of whole vectors on one grid
-    if (g.streaming == 4) return launch_short<DT, false>(p, g, ws, stream);   // short rows of any length anywhere in memory
+    if (g.streaming == 3) return launch_short<DT, kWhole>(p, g, ws, stream);      // short rows of whole vectors on one grid
+    if (g.streaming == 4) return p.seqlen >= vec_elems(p.x_dtype) ? launch_short<DT, kAnywhere>(p, g, ws, stream)   // anywhere in memory
+                                                                  : launch_short<DT, kElements>(p, g, ws, stream);
     if (g.streaming == 1) {                           // rows on the grid, whole vectors
         switch (p.width) {
             case 2: CC1D_LAUNCH((bwd_channelfirst_stream_kernel<DT, 2, false>), dim3(blocks), dim3(kBlock), 0, stream, p, g, ws); break;

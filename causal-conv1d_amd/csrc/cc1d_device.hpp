@@ -232,6 +232,55 @@ __device__ __forceinline__ void st_vec_nt(void *base, int64_t elem_off, const u3
     __builtin_nontemporal_store(
         v, reinterpret_cast<u32x4 *>(reinterpret_cast<T *>(base) + elem_off));
 }
+// A vector that starts at any element: one access wherever the address lies.
+typedef uint32_t u32x4_on2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x4_on4 __attribute__((ext_vector_type(4), aligned(4)));
+template <int DT>
+__device__ __forceinline__ u32x4 ld_vec_any(const void *base, int64_t elem_off) {
+    using T = typename Elem<DT>::type;
+    const T *at = reinterpret_cast<const T *>(base) + elem_off;
+    if constexpr (sizeof(T) == 2) return *reinterpret_cast<const u32x4_on2 *>(at);
+    else return *reinterpret_cast<const u32x4_on4 *>(at);
+}
+// The first n elements (a whole vector or fewer) of v to any element: a vector's front part as one store each
+// of 8, 4 and 2 bytes.  n_front is the same for every lane that stores a front part, so its bits are branches of
+// the wavefront.
+template <int DT>
+__device__ __forceinline__ void st_front_any(void *base, int64_t elem_off, const u32x4 &v, bool whole, int n_front) {
+    using T = typename Elem<DT>::type;
+    typedef uint32_t u32_on2 __attribute__((aligned(2)));
+    typedef uint32_t u32x2_on2 __attribute__((ext_vector_type(2), aligned(2)));
+    T *at = reinterpret_cast<T *>(base) + elem_off;
+    if (whole) {
+        if constexpr (sizeof(T) == 2) *reinterpret_cast<u32x4_on2 *>(at) = v;
+        else *reinterpret_cast<u32x4_on4 *>(at) = v;
+        return;
+    }
+    const int bytes = n_front * (int)sizeof(T);
+    char *to = reinterpret_cast<char *>(at);
+    uint32_t next = v.x, after = v.y;
+    if (bytes & 8) {
+        *reinterpret_cast<u32x2_on2 *>(to) = u32x2_on2{v.x, v.y};
+        to += 8;
+        next = v.z;
+        after = v.w;
+    }
+    if (bytes & 4) {
+        *reinterpret_cast<u32_on2 *>(to) = next;
+        to += 4;
+        next = after;
+    }
+    if (sizeof(T) == 2 && (bytes & 2)) *reinterpret_cast<uint16_t *>(to) = (uint16_t)next;
+}
+// v without its first `bytes` bytes (0 .. 14, even), zeros behind the rest.
+__device__ __forceinline__ u32x4 without_front(const u32x4 &v, int bytes) {
+    const uint32_t x = v.x, y = v.y, z = v.z, w = v.w;   // values: an array here would be chosen from by address, in memory
+    const bool two = (bytes & 8) != 0, one = (bytes & 4) != 0, half = (bytes & 2) != 0;
+    const uint32_t a0 = two ? z : x, a1 = two ? w : y, a2 = two ? 0u : z, a3 = two ? 0u : w;
+    const uint32_t b0 = one ? a1 : a0, b1 = one ? a2 : a1, b2 = one ? a3 : a2, b3 = one ? 0u : a3;
+    return u32x4{half ? __builtin_amdgcn_alignbit(b1, b0, 16) : b0, half ? __builtin_amdgcn_alignbit(b2, b1, 16) : b1,
+                 half ? __builtin_amdgcn_alignbit(b3, b2, 16) : b2, half ? b3 >> 16 : b3};
+}
 template <int DT>
 __device__ __forceinline__ float ld_elem(const void *base, int64_t elem_off) {
     using T = typename Elem<DT>::type;
