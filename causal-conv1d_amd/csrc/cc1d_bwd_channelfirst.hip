@@ -671,7 +671,6 @@ constexpr int kMaxDirectParts = 16;
 // their sums and stores dweight / dbias itself.  The wavefronts take the same rows in the same order as
 // without it; what goes is the second launch, 2-5 us behind a kernel that may run for less (see
 // short_rows_direct for where that is worth it).
-enum ShortRows : int { kWhole, kAnywhere, kElements };
 template <int DT, int W, int ROWS, bool DIRECT>
 __global__ void __launch_bounds__(DIRECT ? kMaxDirectParts * kWave : kBlock)
 bwd_channelfirst_short_kernel(const cc1d_bwd_params p, const BwdCfGeom g, float *__restrict__ ws) {

@@ -232,6 +232,9 @@ __device__ __forceinline__ void st_vec_nt(void *base, int64_t elem_off, const u3
     __builtin_nontemporal_store(
         v, reinterpret_cast<u32x4 *>(reinterpret_cast<T *>(base) + elem_off));
 }
+// How the short-row kernels (channel-first rows of at most 64 vectors) move a row: as whole vectors on the 16-byte
+// grid, as vectors of any address (rows of a vector and more), or element by element.
+enum ShortRows : int { kWhole, kAnywhere, kElements };
 // A vector that starts at any element: one access wherever the address lies.
 typedef uint32_t u32x4_on2 __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x4_on4 __attribute__((ext_vector_type(4), aligned(4)));

@@ -16,7 +16,7 @@
 // initial_states / final_states are supported (the reference refuses them for this
 // layout, csrc/causal_conv1d.cpp:213,228).
 //
-// Four kernels share this design.  The streaming kernel takes every launch in which the rows
+// Three kernels share this design.  The streaming kernel takes every launch in which the rows
 // of out lie on the same 16-byte grid as the rows of x (same shape and strides, as
 // empty_like gives): whole 64-vector steps run without bounds checks in two register sets in
 // ping-pong, which keep the loads of the next two groups in flight while a group is computed
@@ -25,8 +25,7 @@
 // three steps start their steps on 128-byte lines of out, with a partly filled first step; and
 // the few positions of a row in front of its first whole vector or behind its last one are
 // produced one per lane, straight from memory.  The general kernel takes out tensors on a different grid.  The short-row
-// kernel takes rows of at most 64 vectors, several rows to a wavefront and no walk; the flat
-// kernel takes such rows of a contiguous tensor as whole vectors of one flat array.  Rows of
+// kernel takes rows of at most 64 vectors, several rows to a wavefront and no walk.  Rows of
 // more than 64 vectors that start on 128-byte lines (tensors of up to 512 MiB) or hold at most
 // 128 vectors, and rows off the 16-byte grid of up to 512 vectors (192 of fp32), go to the tile
 // kernel of cc1d_fwd_channelfirst_tile.hip (rows fetched straight into LDS; 1-25 % faster on
@@ -442,16 +441,16 @@ fwd_channelfirst_stream_kernel(const cc1d_fwd_params p, const FwdCfGeom g) {
 }
 
 // Rows of at most 64 vectors.  One wavefront per row would leave most of its lanes idle, so a
-// wavefront takes 64 / G rows at once, G = 1, 2, 4 ... 64 lanes each (ALIGNED: whole vectors on the
+// wavefront takes 64 / G rows at once, G = 1, 2, 4 ... 64 lanes each (kWhole: whole vectors on the
 // 16-byte grid): lane (row, v) owns vector v of its row, takes its left halo from the previous lane through the same
 // DPP shift as the walk (vector 0 takes zeros or initial_states instead), and the whole launch is
 // one load and one store per lane.  Same arithmetic, in the same order, as the other kernels.
-// ALIGNED = false: rows of any length up to 64 vectors, anywhere in memory (a contiguous tensor
-// whose seqlen is no multiple of the vector length, down to seqlen 1): the same lanes, with a
-// lane's up to VEC positions read and written element by element.
-template <int DT, int W, bool SILU, bool ALIGNED, bool BI>
+// ROWS: kAnywhere, rows of a vector and more anywhere in memory: the lane of a row's last, partly filled vector
+// reads the row's last 16 bytes, drops what the lane in front of it owns and stores its own part in pieces;
+// kElements, rows shorter than a vector, read and written element by element.
+template <int DT, int W, bool SILU, int ROWS, bool BI>
 __global__ void __launch_bounds__(kBlock)
-fwd_channelfirst_short_kernel(const cc1d_fwd_params p, const int n_vecs, const int lanes_log2, const uint32_t n_rows) {
+fwd_channelfirst_short_kernel(const cc1d_fwd_params p, const int n_vecs, const int lanes_log2, const uint32_t n_rows, const FastDiv by_inner) {
     using E = Elem<DT>;
     using T = typename E::type;
     constexpr int VEC = E::kVec;
@@ -465,15 +464,19 @@ fwd_channelfirst_short_kernel(const cc1d_fwd_params p, const int n_vecs, const i
     // on row 0's addresses; they load and store nothing.
     const bool mine = row_here < n_rows && v < n_vecs;
     const uint32_t row = mine ? row_here : 0u;
-    int b, c;
-    row_to_batch_and_channel<BI>(p, row, b, c);
+    const uint32_t outer = divided(row, by_inner), inner = row - outer * (uint32_t)(BI ? p.batch : p.dim);
+    const int b = (int)(BI ? inner : outer), c = (int)(BI ? outer : inner);
     const int64_t xrow = (int64_t)b * p.x_stride_b + (int64_t)c * p.x_stride_c;
     const int64_t orow = (int64_t)b * p.out_stride_b + (int64_t)c * p.out_stride_c;
 
     const int L = p.seqlen;
+    // kAnywhere: how many bytes of the row's last 16 the lane of its last vector shares with the lane in front of it.
+    const int shared = ROWS == kAnywhere && v == n_vecs - 1 ? (n_vecs * VEC - L) * E::kBytes : 0;
     u32x4 raw = u32x4{0u, 0u, 0u, 0u};
-    if (ALIGNED) {
+    if (ROWS == kWhole) {
         if (mine) raw = ld_vec_nt<DT>(p.x, xrow + (int64_t)v * VEC);
+    } else if (ROWS == kAnywhere) {
+        if (mine) raw = ld_vec_any<DT>(p.x, xrow + v * VEC - shared / E::kBytes);
     } else {
         T elems[VEC];
 #pragma unroll
@@ -501,7 +504,7 @@ fwd_channelfirst_short_kernel(const cc1d_fwd_params p, const int n_vecs, const i
     }
 
     float xf[VEC];
-    E::unpack(raw, xf);
+    E::unpack(ROWS == kAnywhere ? without_front(raw, shared) : raw, xf);
     float xx[VEC + W - 1];
 #pragma unroll
     for (int i = 0; i < W - 1; ++i) {
@@ -518,8 +521,10 @@ fwd_channelfirst_short_kernel(const cc1d_fwd_params p, const int n_vecs, const i
         for (int w = 0; w < W; ++w) a = fmaf(wv[w], xx[e + w], a);
         acc[e] = SCALED ? silu_from_scaled(a) : SILU ? silu<PRECISE>(a) : a;
     }
-    if (ALIGNED) {
+    if (ROWS == kWhole) {
         if (mine) st_vec_nt<DT>(p.out, orow + (int64_t)v * VEC, E::pack(acc));
+    } else if (ROWS == kAnywhere) {
+        if (mine) st_front_any<DT>(p.out, orow + v * VEC, E::pack(acc), shared == 0, VEC - (n_vecs * VEC - L));
     } else if (mine) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e)
@@ -561,11 +566,14 @@ int launch_short(const cc1d_fwd_params &p, int n_vecs, bool aligned, hipStream_t
     const dim3 grid((uint32_t)((threads + kBlock - 1) / kBlock)), block(kBlock);
     const uint32_t n_rows = (uint32_t)rows;
     const bool batch_inner = batch_entries_are_neighbours(p);
-#define CC1D_SHORT3(WIDTH, SILU_ON, BI_ON)                                                                           \
-    if (aligned) CC1D_LAUNCH((fwd_channelfirst_short_kernel<DT, WIDTH, SILU_ON, true, BI_ON>), grid, block, 0, \
-                                    stream, p, n_vecs, lanes_log2, n_rows);                                           \
-    else CC1D_LAUNCH((fwd_channelfirst_short_kernel<DT, WIDTH, SILU_ON, false, BI_ON>), grid, block, 0,       \
-                            stream, p, n_vecs, lanes_log2, n_rows)
+    const FastDiv by_inner = fast_div((uint32_t)(batch_inner ? p.batch : p.dim));
+#define CC1D_SHORT4(WIDTH, SILU_ON, BI_ON, ROWS)                                                                      \
+    CC1D_LAUNCH((fwd_channelfirst_short_kernel<DT, WIDTH, SILU_ON, ROWS, BI_ON>), grid, block, 0, stream, p, n_vecs,  \
+                lanes_log2, n_rows, by_inner)
+#define CC1D_SHORT3(WIDTH, SILU_ON, BI_ON)                                                                            \
+    if (aligned) CC1D_SHORT4(WIDTH, SILU_ON, BI_ON, kWhole);                                                          \
+    else if (p.seqlen >= vec_elems(DT)) CC1D_SHORT4(WIDTH, SILU_ON, BI_ON, kAnywhere);                                \
+    else CC1D_SHORT4(WIDTH, SILU_ON, BI_ON, kElements)
 #define CC1D_SHORT2(WIDTH, SILU_ON)                                                                                  \
     if (batch_inner) { CC1D_SHORT3(WIDTH, SILU_ON, true); } else { CC1D_SHORT3(WIDTH, SILU_ON, false); }
 #define CC1D_SHORT(WIDTH)                                                                                             \
@@ -578,159 +586,7 @@ int launch_short(const cc1d_fwd_params &p, int n_vecs, bool aligned, hipStream_t
 #undef CC1D_SHORT
 #undef CC1D_SHORT2
 #undef CC1D_SHORT3
-    return launch_status();
-}
-
-// Short rows of a contiguous tensor whose seqlen is no multiple of the vector length (at least
-// one vector, at most 64): rows then start anywhere on the 16-byte grid, but batch * dim * seqlen
-// elements lie back to back, so a lane owns one whole vector of that flat array: one 16-byte load
-// and one 16-byte store, as in the short-row kernel, where element accesses would take VEC of each.
-// A vector spans at most two rows; the lane holds the taps of both, takes its left neighbours from
-// the previous lane (lane 0 of a wavefront from memory) and masks the taps that reach in front of
-// a row's start (or takes initial_states there).  Same arithmetic, in the same order, as the
-// other kernels.
-template <int DT, int W, bool SILU, bool PACKED_W>
-__global__ void __launch_bounds__(kBlock)
-fwd_channelfirst_flat_kernel(const cc1d_fwd_params p, const uint32_t n_elems) {
-    using E = Elem<DT>;
-    using T = typename E::type;
-    constexpr int VEC = E::kVec;
-    constexpr bool PRECISE = E::kPreciseAct;
-    constexpr bool SCALED = SILU && !PRECISE;
-
-    const uint32_t gid = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
-    const int lane = threadIdx.x & (kWave - 1);
-    const uint32_t L = (uint32_t)p.seqlen, D = (uint32_t)p.dim;
-    // Lanes past the end stay in step (the lane shift needs every lane) on vector 0.
-    const bool mine = (uint64_t)gid * VEC < n_elems;
-    const uint32_t f0 = mine ? gid * VEC : 0u;
-    const bool whole = f0 + VEC <= n_elems;           // only the array's last vector can be partial
-
-    u32x4 raw = u32x4{0u, 0u, 0u, 0u};
-    if (mine) {
-        if (whole) {
-            raw = ld_vec_nt<DT>(p.x, f0);
-        } else {
-            T elems[VEC];
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) elems[e] = f0 + e < n_elems ? ld_raw<DT>(p.x, f0 + e) : T(0.f);
-            __builtin_memcpy(&raw, elems, sizeof raw);
-        }
-    }
-    const uint32_t row0 = f0 / L;
-    const uint32_t t0 = f0 - row0 * L;
-    const uint32_t split = L - t0;                    // elements [split, VEC) belong to the next row
-    const uint32_t c0 = row0 % D, b0 = row0 / D;
-    const bool wrap = c0 + 1 == D;
-    const uint32_t c1 = wrap ? 0u : c0 + 1, b1 = wrap ? b0 + 1 : b0;
-
-    // Taps of the row the vector starts in, and of the next one only where the vector reaches it
-    // (one lane in seqlen / VEC).  Packed fp32 taps (a host-checked promise: strides (W, 1), base
-    // 16-byte aligned) of even width come in one load.
-    float w0[W], w1[W], bias0, bias1 = 0.f;
-    auto taps = [&](uint32_t c, float (&wv)[W], float &bv) {
-        if (PACKED_W && W % 2 == 0) {
-            const float *src = static_cast<const float *>(__builtin_assume_aligned(
-                reinterpret_cast<const float *>(p.weight) + (int64_t)c * W, W % 2 == 0 ? W * 4 : 4));
-#pragma unroll
-            for (int w = 0; w < W; ++w) wv[w] = src[w];
-            bv = p.bias == nullptr ? 0.f : reinterpret_cast<const float *>(p.bias)[c];   // of the taps' type
-        } else {
-            channel_taps<W>(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, (int)c, wv, bv);
-        }
-    };
-    taps(c0, w0, bias0);
-#pragma unroll
-    for (int w = 0; w < W; ++w) w1[w] = 0.f;
-    if (split < (uint32_t)VEC) taps(c1, w1, bias1);
-    if (SCALED) {
-        bias0 *= kSiluPrescale;
-        bias1 *= kSiluPrescale;
-#pragma unroll
-        for (int w = 0; w < W; ++w) { w0[w] *= kSiluPrescale; w1[w] *= kSiluPrescale; }
-    }
-
-    float xf[VEC];
-    E::unpack(raw, xf);
-    // xx[i] = flat element f0-(W-1)+i
-    float xx[VEC + W - 1];
-    float first[W - 1];
-#pragma unroll
-    for (int i = 0; i < W - 1; ++i) first[i] = 0.f;
-    if (lane == 0 && f0 >= (uint32_t)(W - 1)) {
-#pragma unroll
-        for (int i = 0; i < W - 1; ++i) first[i] = ld_elem<DT>(p.x, (int64_t)f0 - (W - 1) + i);
-    }
-#pragma unroll
-    for (int i = 0; i < W - 1; ++i) xx[i] = from_prev_lane(xf[VEC - (W - 1) + i], first[i]);
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) xx[W - 1 + e] = xf[e];
-
-    const bool has_init = p.initial_states != nullptr;
-    float acc[VEC];
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-        const bool next = (uint32_t)e >= split;
-        const uint32_t t = next ? (uint32_t)e - split : t0 + (uint32_t)e;
-        float a = next ? bias1 : bias0;
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            // tap w reads position t-(W-1-w) of the row
-            float xv = xx[e + w];
-            if (w < W - 1 && t + (uint32_t)w < (uint32_t)(W - 1)) {
-                xv = 0.f;
-                if (has_init && f0 + e < n_elems)     // (positions past the array's end belong to no row)
-                    xv = ld_elem<DT>(p.initial_states, (int64_t)(next ? b1 : b0) * p.init_stride_b +
-                                                           (int64_t)(next ? c1 : c0) * p.init_stride_c +
-                                                           (int64_t)(t + w) * p.init_stride_l);
-            }
-            a = fmaf(next ? w1[w] : w0[w], xv, a);
-        }
-        acc[e] = SCALED ? silu_from_scaled(a) : SILU ? silu<PRECISE>(a) : a;
-    }
-    if (mine) {
-        if (whole) {
-            st_vec_nt<DT>(p.out, f0, E::pack(acc));
-        } else {
-#pragma unroll
-            for (int e = 0; e < VEC; ++e)
-                if (f0 + e < n_elems) st_elem<DT>(p.out, f0 + e, acc[e]);
-        }
-    }
-
-    // final_states[b, c, i] = x[L-(W-1)+i] (a row is never shorter than a vector, so never
-    // shorter than W-1), bit-exact copies, by the lane whose vector holds the row's last element.
-    if (p.final_states != nullptr && mine && split <= (uint32_t)VEC && f0 + split <= n_elems) {
-#pragma unroll
-        for (int i = 0; i < W - 1; ++i) {
-            const T e = ld_raw<DT>(p.x, (int64_t)f0 + split - (W - 1) + i);
-            st_raw<DT>(p.final_states, (int64_t)b0 * p.final_stride_b + (int64_t)c0 * p.final_stride_c +
-                                           (int64_t)i * p.final_stride_l, e);
-        }
-    }
-}
-
-template <int DT>
-int launch_flat(const cc1d_fwd_params &p, hipStream_t stream) {
-    constexpr int VEC = Elem<DT>::kVec;
-    const uint32_t n_elems = (uint32_t)((int64_t)p.batch * p.dim * p.seqlen);
-    const uint32_t n_vecs = (n_elems + VEC - 1) / VEC;
-    const dim3 grid((n_vecs + kBlock - 1) / kBlock), block(kBlock);
-    const bool packed = weights_contiguous_f32(p.weight, p.w_dtype, p.w_stride_c, p.w_stride_w, p.width);
-#define CC1D_FLAT2(WIDTH, SILU_ON)                                                                                    \
-    if (packed) CC1D_LAUNCH((fwd_channelfirst_flat_kernel<DT, WIDTH, SILU_ON, true>), grid, block, 0, stream,  \
-                                   p, n_elems);                                                                       \
-    else CC1D_LAUNCH((fwd_channelfirst_flat_kernel<DT, WIDTH, SILU_ON, false>), grid, block, 0, stream, p,     \
-                            n_elems)
-#define CC1D_FLAT(WIDTH)                                                                                              \
-    if (p.silu) { CC1D_FLAT2(WIDTH, true); } else { CC1D_FLAT2(WIDTH, false); }
-    switch (p.width) {
-        case 2: CC1D_FLAT(2); break;
-        case 3: CC1D_FLAT(3); break;
-        default: CC1D_FLAT(4); break;
-    }
-#undef CC1D_FLAT
-#undef CC1D_FLAT2
+#undef CC1D_SHORT4
     return launch_status();
 }
 
@@ -790,31 +646,17 @@ int launch_fwd_channelfirst(const cc1d_fwd_params &p, hipStream_t stream) {
     const int64_t rows = (int64_t)p.batch * p.dim;
     // Short rows of whole vectors, up to eight to a wavefront, no walk: (4, 5376, 256) bf16 11.2 -> 6.0 us,
     // (8, 1024, 512) bf16 6.7 -> 4.8 us, (4, 5376, 256) fp32 10.9 -> 8.5 us, (1, 5376, 64) bf16 4.8 -> 3.3 us.
-    // Rows that are not whole vectors on one grid take the same lanes with element accesses:
-    // (16, 5376, 100) bf16 45.9 -> 25.4 us, (64, 2048, 60) 63.7 -> 16.4 us, (256, 5376, 4) 360 -> 11.9 us.
+    // Rows that are not whole vectors on one grid take the same lanes, vectors of any address and the last one of
+    // a row in pieces, or single elements where a row is shorter than a vector.  Against whole vectors of the flat
+    // array, each with the taps of the two rows it may span (contiguous tensors; others took elements):
+    // (8, 4096, 500) bf16 22.6 -> 14.8 us, (16, 5376, 100) 14.8 -> 10.8, (64, 2048, 60) 12.8 -> 9.0, (4, 1024, 300) 5.1 -> 3.4,
+    // (32, 4096, 250) 42.9 -> 25.6, (8, 2048, 250) fp32 10.4 -> 9.0, and where half of the lanes have no vector
+    // (16, 2048, 265) 15.4 -> 14.0, (16, 5376, 130) 17.2 -> 16.0; (3, 6000, 77) with states 7.4 -> 5.0.
+    // (256, 5376, 4) 360 -> 11.9 us walking -> elements.
     const int64_t short_vecs = ((int64_t)p.seqlen + vec - 1) / vec;
     const int32_t forced_vecs = tunables().fwd_cf_vecs;
     if (short_vecs <= 64 && forced_vecs <= 0) {
         const bool aligned = same_grid && on_grid && p.seqlen % vec == 0;
-        // A contiguous tensor of rows that are not whole vectors, but at least one: whole vectors of
-        // the flat array, (16, 5376, 100) bf16 25.4 -> 13.5 us, (16, 5376, 130) 28.5 -> 16.2 us, (64, 2048, 60) 16.4 -> 11.6 us.
-        const int64_t n_elems = rows * p.seqlen;
-        // (Not when final_states may be the buffer initial_states come from: in the flat walk the
-        // lane that reads a row's initial_states and the lane that writes its final_states can sit in
-        // different wavefronts.)
-        const bool states_in_and_out = p.initial_states != nullptr && p.final_states != nullptr;
-        const bool flat = !aligned && !states_in_and_out && p.seqlen >= vec && n_elems < thread_limit() &&
-                          aligned16(p.x) && aligned16(p.out) &&
-                          (p.dim == 1 || (p.x_stride_c == p.seqlen && p.out_stride_c == p.seqlen)) &&
-                          (p.batch == 1 || (p.x_stride_b == (int64_t)p.dim * p.seqlen &&
-                                            p.out_stride_b == (int64_t)p.dim * p.seqlen));
-        if (flat) {
-            switch (p.x_dtype) {
-                case CC1D_F32: return launch_flat<CC1D_F32>(p, stream);
-                case CC1D_F16: return launch_flat<CC1D_F16>(p, stream);
-                default: return launch_flat<CC1D_BF16>(p, stream);
-            }
-        }
         switch (p.x_dtype) {
             case CC1D_F32: return launch_short<CC1D_F32>(p, (int)short_vecs, aligned, stream);
             case CC1D_F16: return launch_short<CC1D_F16>(p, (int)short_vecs, aligned, stream);

@@ -48,3 +48,33 @@ def test_rows_anywhere(pkg, gpu_device, dtype, seqlen, batch, dim, width, states
         assert_close(dinit, ref[3], dtype, "dinitial_states")
     dx.fill_(7.0)
     assert bool((buf == 7.0).all())
+
+
+@pytest.mark.parametrize("dense", [True, False], ids=["contiguous", "apart"])
+@pytest.mark.parametrize("states", [False, True], ids=["plain", "states"])
+@pytest.mark.parametrize("batch,dim,width,silu", [(3, 40, 4, True), (24, 16, 3, False), (2, 1032, 2, True)])
+@pytest.mark.parametrize("dtype,seqlen", CASES, ids=["%s-%d" % (str(d)[6:], n) for d, n in CASES])
+def test_forward_of_rows_anywhere(pkg, gpu_device, dtype, seqlen, batch, dim, width, silu, states, dense):
+    """The forward of the same rows, one buffer for initial and final states."""
+    g = gen(2000 * width + seqlen)
+    apart, start = (seqlen, 0) if dense else (seqlen + (3 if seqlen % 2 else 2), 5)
+
+    def spread():
+        buf = torch.full((start + batch * dim * apart + 8,), 7.0, dtype=dtype, device=gpu_device)
+        return buf, buf.as_strided((batch, dim, seqlen), (dim * apart, apart, 1), start)
+
+    x = torch.randn(batch, dim, seqlen, generator=g).to(dtype)
+    w, b = make_wb(dim, width, True, g)
+    init = make_states(batch, dim, width - 1, dtype, g) if states else None
+    _, xg = spread()
+    xg.copy_(x)
+    buf, out = spread()
+    held = init.to(gpu_device) if states else None
+    torch.ops.DaoAILab._causal_conv1d_fwd_cpp(xg, w.to(gpu_device), b.to(gpu_device), None, held, out, held, silu)
+    ref = orc.fwd(x, w, b, initial_states=init, return_final_states=states, activation="silu" if silu else None)
+    ref, fin = ref if states else (ref, None)
+    assert_close(out, ref, dtype, "out")
+    if states:
+        assert torch.equal(held.cpu(), fin)
+    out.fill_(7.0)
+    assert bool((buf == 7.0).all())
