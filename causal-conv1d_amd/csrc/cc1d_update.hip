@@ -4,7 +4,7 @@
 // Four kernels:
 //  * update_step_kernel — the decode step proper: one new token (seqlen 1) and x, out,
 //    conv_state with unit stride along dim.  A lane owns one 8-byte vector of channels of
-//    two consecutive batch entries; all of its loads (window rows, x) are issued before
+//    one batch entry, or of two consecutive ones (two_step_rows); all of its loads (window rows, x) are issued before
 //    anything is consumed, the taps come through LDS once per workgroup, and the grid is
 //    (column blocks, batch blocks), so no index division sits in front of the first load.
 //    This shape moves about 22 MB; its
@@ -754,10 +754,22 @@ bool rows_lane_ok(const void *ptr, int dtype, int lane_bytes, int64_t sb, int64_
 }
 
 constexpr int kStepLaneBytes = 8;
-#ifndef CC1D_UPDATE_STEP_ROWS
-#define CC1D_UPDATE_STEP_ROWS 2
-#endif
-constexpr int kStepRows = CC1D_UPDATE_STEP_ROWS;   // batch rows per lane
+constexpr int kStepRowsMax = 2;                    // batch rows per lane: one or two
+
+// One, except in a launch that two rows a lane bring to just under two workgroups for each of the 256 CUs: one
+// row a lane would then be just under four, twice the workgroups for the same evenness.  Everywhere else one row
+// has the shorter chain and twice the wavefronts in flight.  us a launch over 40 rotating sets, two rows / one row
+// (workgroups with two rows): bf16 batch 8, dim 5376, state 4 (21) 2.72 / 2.42; 32 (84) 2.96 / 2.73; (128, 5376, 3) (336)
+// 4.11 / 3.69; (256, 2560, 3) (320) 4.09 / 3.68; fp32 (64, 5376, 4) in 128 slots (336) 4.24 / 3.85; (224, 5376, 3) (588)
+// 5.44 / 5.26; (256, 5376, 3) (672) 5.74 / 5.75; (512, 2560, 3) (640) 5.63 / 5.69; (512, 5376, 4) (1344) 10.85 / 10.56;
+// (1024, 5376, 3) (2688) 16.79 / 16.51; and kept at two, ring fp16 (384, 2560, 8) (480) 4.12 / 4.17, (192, 5376, 4) (504)
+// 4.89 / 5.06, fp32 (96, 5376, 3) (504) 4.38 / 4.56, (256, 4096, 3) (512) 4.50 / 4.55.  Three and four rows are
+// slower at every size.
+bool two_step_rows(int64_t column_blocks, int64_t batch) {
+    const int64_t two = column_blocks * ((batch + 2 * kStepWaves - 1) / (2 * kStepWaves));
+    const int64_t one = column_blocks * ((batch + kStepWaves - 1) / kStepWaves);
+    return (two > 448 && two <= 512) || one * kBlock >= thread_limit();
+}
 
 template <int DT, int W>
 int launch_w(const cc1d_update_params &p, bool vec, hipStream_t stream) {
@@ -766,7 +778,7 @@ int launch_w(const cc1d_update_params &p, bool vec, hipStream_t stream) {
     // Taps packed (dim, W) in fp32 or in x's own type, as callers in practice pass them;
     // anything else takes the general kernels below.
     const int mode = weights_mode(p.weight, p.bias, p.w_dtype, DT, p.w_stride_c, p.w_stride_w, p.width);
-    const bool step = p.seqlen == 1 && p.dim % CH == 0 && p.batch <= 65535 * kStepRows && mode != 0 &&
+    const bool step = p.seqlen == 1 && p.dim % CH == 0 && p.batch <= 65535 * kStepRowsMax && mode != 0 &&
         rows_lane_ok(p.x, DT, kStepLaneBytes, p.x_stride_b, p.x_stride_c, p.x_stride_l, 1) &&
         rows_lane_ok(p.out, DT, kStepLaneBytes, p.out_stride_b, p.out_stride_c, p.out_stride_l, 1) &&
         rows_lane_ok(p.conv_state, DT, kStepLaneBytes, p.state_stride_b, p.state_stride_c, p.state_stride_l, p.state_len);
@@ -780,17 +792,22 @@ int launch_w(const cc1d_update_params &p, bool vec, hipStream_t stream) {
         a.state_stride_b = p.state_stride_b; a.state_stride_l = p.state_stride_l;
         a.batch = p.batch; a.state_len = p.state_len;
         a.n_colgroups = (uint32_t)(p.dim / CH);
-        const dim3 grid((a.n_colgroups + kWave - 1) / kWave,
-                        (uint32_t)((p.batch + kStepWaves * kStepRows - 1) / (kStepWaves * kStepRows)));
+        const uint32_t column_blocks = (a.n_colgroups + kWave - 1) / kWave;
+        const bool two_rows = two_step_rows(column_blocks, p.batch);
+        const int block_rows = kStepWaves * (two_rows ? 2 : 1);
+        const dim3 grid(column_blocks, (uint32_t)((p.batch + block_rows - 1) / block_rows));
         if ((int64_t)grid.x * grid.y * kBlock >= thread_limit()) return CC1D_ERR_TOO_LARGE;
         auto launch = [&](auto wm) {
             constexpr int WM = decltype(wm)::value;
+            auto run = [&](auto ring, auto act) {
+                constexpr bool CIRC = decltype(ring)::value, SILU = decltype(act)::value;
+                if (two_rows) CC1D_LAUNCH((update_step_kernel<DT, CH, W, CIRC, SILU, 2, WM>), grid, dim3(kBlock), 0, stream, a);
+                else CC1D_LAUNCH((update_step_kernel<DT, CH, W, CIRC, SILU, 1, WM>), grid, dim3(kBlock), 0, stream, a);
+            };
             if (circ) {
-                if (p.silu) CC1D_LAUNCH((update_step_kernel<DT, CH, W, true, true, kStepRows, WM>), grid, dim3(kBlock), 0, stream, a);
-                else CC1D_LAUNCH((update_step_kernel<DT, CH, W, true, false, kStepRows, WM>), grid, dim3(kBlock), 0, stream, a);
+                if (p.silu) run(std::true_type{}, std::true_type{}); else run(std::true_type{}, std::false_type{});
             } else {
-                if (p.silu) CC1D_LAUNCH((update_step_kernel<DT, CH, W, false, true, kStepRows, WM>), grid, dim3(kBlock), 0, stream, a);
-                else CC1D_LAUNCH((update_step_kernel<DT, CH, W, false, false, kStepRows, WM>), grid, dim3(kBlock), 0, stream, a);
+                if (p.silu) run(std::false_type{}, std::true_type{}); else run(std::false_type{}, std::false_type{});
             }
         };
         if (mode == 1) launch(std::integral_constant<int, 1>{});
