@@ -186,8 +186,8 @@ def test_decode_step_in_batch_slices(pkg, gpu_device, cc1d_lib, layout, circular
 
 
 def test_flat_forward_in_batch_slices(pkg, gpu_device, cc1d_lib):
-    """Contiguous channel-first rows that are no whole number of vectors (the flat kernel reads the
-    tensor as one array): sliced along the batch against the single launch."""
+    """Contiguous channel-first rows that are no whole number of vectors: sliced along the batch against
+    the single launch."""
     lib = cabi.declare(cc1d_lib)
     dev = gpu_device
     g = gen(92)

@@ -94,9 +94,9 @@ def test_fwd_channel_first_short_rows(pkg, gpu_device, seqlen, dtype):
 def test_fwd_channel_first_short_rows_of_any_length(pkg, gpu_device, seqlen, dtype):
     """Channel-first rows of at most 64 vectors that are not whole vectors (a contiguous tensor
     whose seqlen is no multiple of 16 bytes) share wavefronts too, down to one lane per row; rows
-    shorter than width-1 take part of final_states from initial_states (or zeros).  Contiguous
-    tensors with rows of at least one vector are walked as one flat array of whole vectors, a
-    vector spanning two rows; slices of a wider tensor take element accesses."""
+    shorter than width-1 take part of final_states from initial_states (or zeros).  Rows of at
+    least one vector move as vectors of any address, contiguous or slices of a wider tensor, the last one
+    in pieces; shorter rows take element accesses."""
     dev = gpu_device
     batch, dim = 3, 41                                 # batch * dim * seqlen is no whole number of vectors either
     for width in (2, 3, 4):
