@@ -376,13 +376,17 @@ int launch_taps(const FwdClArgs &a, const FwdClRare &q, int width, bool silu, in
 // holds, and hold less LDS, so more of them are in flight.  Measured at the prefill shape
 // (8, 5376, 2048) bf16, the same buffers every launch / six rotating sets: 8 rows 64.7 / 62.7 us,
 // 16 rows 56.1 / 55.9, 24 rows 57.8 / 57.5, 32 rows 58.5 / 58.3.
-// Launches of at most 1536 wavefronts (a fifth of what the chip holds: a prompt of a few dozen
-// tokens, a short chunk of a prefill) are bound by one wavefront's chain of fetch, walk and store
-// and take runs of 8 rows: (1, 5376, 64) bf16 4.65 -> 4.05 us, (4, 5376, 128) 5.19 -> 4.70,
-// (1, 5376, 512) 5.16 -> 4.65; at 2048 wavefronts and more 16 rows are as fast or faster.
+// Launches of at most 1600 wavefronts (400 workgroups: a prompt of a few dozen tokens, a short chunk of a
+// prefill) are bound by one wavefront's chain of fetch, walk and store and take runs of 8 rows: (1, 5376, 64) bf16
+// 4.65 -> 4.05 us, (4, 5376, 128) 5.19 -> 4.70, (1, 5376, 512) 5.16 -> 4.65, (4, 816, 878) 5.58 -> 5.16.  So do those of
+// just over two 16-row workgroups for each of the 256 CUs, which wait for the few CUs that hold a third: us with
+// 16 / 8 rows (workgroups), cold buffers, bf16 (1, 1520, 2767) 7.02 / 6.72 (519), (24, 640, 288) 6.89 / 6.41 (540),
+// (2, 352, 6320) 7.05 / 6.68 (593), fp32 (13, 3776, 40) with seq_idx 6.33 / 5.68 (576).  In between 16 rows are as fast ((1, 672, 4976) 5.37 /
+// 5.41 (467), fp32 (2, 1088, 907) 5.44 / 5.63 (485)), from 640 workgroups on faster ((1, 2152, 1208) fp32 6.79 / 7.35 (646)).  70
+// shapes of every type and alignment in these two ranges: 5 % on average, none slower than 0.3 %.
 static int choose_rows_per_run(int seqlen, int64_t row_bytes, int width, int64_t waves_at_default) {
     int T = tunables().fwd_cl_rows;
-    if (T <= 0) T = waves_at_default <= 1536 ? kGroup : kDefaultRows;
+    if (T <= 0) T = waves_at_default <= 1600 || (waves_at_default > 2048 && waves_at_default <= 2500) ? kGroup : kDefaultRows;
     const int cap = (seqlen + kGroup - 1) / kGroup * kGroup;      // never longer than the sequence
     if (T > cap) T = cap;
     T = (T + kGroup - 1) / kGroup * kGroup;
