@@ -591,8 +591,13 @@ Gradients backward_tensors(const at::Tensor &x, const at::Tensor &weight, const 
 std::optional<at::Tensor> if_defined(const at::Tensor &t) { return t.defined() ? std::optional<at::Tensor>(t) : std::nullopt; }
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
-template <bool SILU, bool FINAL>
-struct CausalConv1dFn : public torch::autograd::Function<CausalConv1dFn<SILU, FINAL>> {
+// How: activation, final states returned, gradient of initial_states wanted.  The last is settled in the forward,
+// like the others: the tensor that the backward unpacks may have been detached in between, or come back from
+// saved-tensor hooks or a checkpoint without requires_grad.
+enum Graph : int { kSilu = 1, kFinal = 2, kDinit = 4 };
+template <int HOW>
+struct CausalConv1dFn : public torch::autograd::Function<CausalConv1dFn<HOW>> {
+    static constexpr bool SILU = (HOW & kSilu) != 0, FINAL = (HOW & kFinal) != 0, DINIT = (HOW & kDinit) != 0;
     static constexpr bool is_traceable = true;        // compiled autograd: the backward is dispatcher calls only
     static variable_list forward(AutogradContext *ctx, const at::Tensor &x, const at::Tensor &weight, const std::optional<at::Tensor> &bias,
                                  const std::optional<at::Tensor> &seq_idx, const std::optional<at::Tensor> &init) {
@@ -609,13 +614,20 @@ struct CausalConv1dFn : public torch::autograd::Function<CausalConv1dFn<SILU, FI
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
         const variable_list saved = ctx->get_saved_variables();
-        const at::Tensor &x = saved[0], &weight = saved[1], &init = saved[4];
+        const at::Tensor &x = saved[0], &weight = saved[1];
         const at::Tensor dout = kernel_layout(grads[0]) ? grads[0] : grads[0].contiguous();
-        Gradients g = backward_tensors(x, weight, if_defined(saved[2]), dout, if_defined(saved[3]), if_defined(init),
-                                       FINAL ? if_defined(grads[1]) : std::nullopt, init.defined() && init.requires_grad(), SILU);
+        Gradients g = backward_tensors(x, weight, if_defined(saved[2]), dout, if_defined(saved[3]), if_defined(saved[4]),
+                                       FINAL ? if_defined(grads[1]) : std::nullopt, DINIT, SILU);
         return {g.dx, g.dweight, g.dbias.value_or(at::Tensor()), at::Tensor(), g.dinit.value_or(at::Tensor())};
     }
 };
+template <int HOW>
+variable_list recorded(const at::Tensor &x, const at::Tensor &weight, const std::optional<at::Tensor> &bias,
+                       const std::optional<at::Tensor> &seq_idx, const std::optional<at::Tensor> &init) {
+    return CausalConv1dFn<HOW>::apply(x, weight, bias, seq_idx, init);
+}
+constexpr decltype(&recorded<0>) recorders[] = {recorded<0>, recorded<1>, recorded<2>, recorded<3>,
+                                                recorded<4>, recorded<5>, recorded<6>, recorded<7>};
 // What only the Python function answers for: functorch transforms and forward-mode gradients, which it refuses in its own words.
 bool python_graph_needed(const std::optional<at::Tensor> &t) { return t.has_value() && (t->has_names() || t->_fw_grad(0).defined()); }
 
@@ -641,10 +653,8 @@ PyObject *forward_call(PyObject *, PyObject *const *a, Py_ssize_t n) {
                                        (init.has_value() && init->requires_grad()))) {
         if (fin.has_value() || functorch_active() || python_graph_needed(x) || python_graph_needed(weight) || python_graph_needed(bias) || python_graph_needed(init))
             NOT_IMPLEMENTED();
-        variable_list res = return_final ? (silu ? CausalConv1dFn<true, true>::apply(x, weight, bias, seq_idx, init)
-                                                 : CausalConv1dFn<false, true>::apply(x, weight, bias, seq_idx, init))
-                                         : (silu ? CausalConv1dFn<true, false>::apply(x, weight, bias, seq_idx, init)
-                                                 : CausalConv1dFn<false, false>::apply(x, weight, bias, seq_idx, init));
+        const bool dinit = init.has_value() && init->requires_grad();
+        variable_list res = recorders[(silu ? kSilu : 0) | (return_final ? kFinal : 0) | (dinit ? kDinit : 0)](x, weight, bias, seq_idx, init);
         out = std::move(res[0]);
         if (return_final) fin = std::move(res[1]);
     } else {

@@ -1,8 +1,12 @@
 """The graph that `causal_conv1d_fn` records from C++ against the one of `CausalConv1dFn`, the Python function:
-which of the two a call takes, that hooks and checkpoints see the same tensors in both, and that the
-gradients are the same bits, also for inputs without gradients, outputs without one and a second pass."""
+which of the two a call takes, that hooks and checkpoints see the same tensors in both, that every input gets its
+gradient whatever happens to the saved tensors in between, and that the gradients are the same bits, also for inputs
+without gradients, outputs without one and a second pass."""
+import contextlib
+
 import pytest
 import torch
+from torch._dynamo import compiled_autograd
 from torch.utils.checkpoint import checkpoint
 
 from helpers import gen, make_states, make_wb, make_x, random_seq_idx, to_dev_like
@@ -77,6 +81,35 @@ def test_hooks_and_second_order(pkg, monkeypatch):
     assert native == python and len(native[0]) == 6
 
 
+@pytest.mark.parametrize("compiled", [False, True], ids=["engine", "compiled_autograd"])
+@pytest.mark.parametrize("between", ["nothing", "hooks", "checkpoint", "reentrant", "detached"])
+def test_every_gradient_arrives(pkg, monkeypatch, between, compiled):
+    """On meta tensors, without a GPU: what happens to initial_states between forward and backward (saved-tensor hooks
+    that hand back another tensor, a checkpoint's second forward, an in-place detach) takes no gradient away.
+    initial_states are a leaf, or in front of one."""
+    if between == "reentrant" and compiled:
+        pytest.skip("a reentrant checkpoint runs the engine inside of the engine")
+
+    def run(leaf):
+        leaves = [_meta(2, 8, 9, grad=True), _meta(8, 4, grad=True), _meta(8, grad=True), _meta(2, 8, 3, grad=True)]
+        init = leaves[3] if leaf else leaves[3] * 2
+        f = lambda x, w, b, i: pkg.causal_conv1d_fn(x, w, b, initial_states=i, return_final_states=True, activation="silu")
+        hooks = torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach(), lambda t: t) if between == "hooks" else contextlib.nullcontext()
+        with hooks:
+            if between in ("checkpoint", "reentrant"):
+                out, fin = checkpoint(f, *leaves[:3], init, use_reentrant=between == "reentrant")
+            else:
+                out, fin = f(*leaves[:3], init)
+        if between == "detached" and not leaf:
+            init.detach_()
+        with compiled_autograd._enable(torch.compile(backend="eager")) if compiled else contextlib.nullcontext():
+            (out.sum() + fin.sum()).backward()
+        return [None if t.grad is None else tuple(t.grad.shape) for t in leaves]
+
+    native, python = _both(monkeypatch, lambda: (run(True), run(False)))
+    assert native == python == ([(2, 8, 9), (8, 4), (8,), (2, 8, 3)],) * 2
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("channel_last", [False, True], ids=["cf", "cl"])
 @pytest.mark.parametrize("extra", ["none", "states", "seq_idx", "no_bias"])
@@ -107,7 +140,10 @@ def test_both_graphs_give_the_same(pkg, gpu_device, monkeypatch, channel_last, e
 
     def everything():
         res = run() + run((True, False, False, False)) + run((False, True, False, False))
-        res += run(through=lambda f, *a: checkpoint(f, *a, use_reentrant=False)) if init is None else run(final_only=True)
+        res += run(through=lambda f, *a: checkpoint(f, *a, use_reentrant=False))
+        if init is not None:
+            res += run((False, False, False, True)) + run(final_only=True)
+            res += run(final_only=True, through=lambda f, *a: checkpoint(f, *a, use_reentrant=False))
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):
