@@ -110,6 +110,13 @@ def test_every_gradient_arrives(pkg, monkeypatch, between, compiled):
     assert native == python == ([(2, 8, 9), (8, 4), (8,), (2, 8, 3)],) * 2
 
 
+def test_gradient_of_states_that_need_a_copy(pkg):
+    """On meta tensors, without a GPU: initial_states with no unit stride are copied first, and keep their gradient."""
+    x, w, init = _meta(2, 8, 9, grad=True), _meta(8, 4), _meta(2, 16, 6, grad=True)
+    pkg.causal_conv1d_fn(x, w, initial_states=init[:, ::2, ::2]).sum().backward()
+    assert x.grad.shape == x.shape and init.grad is not None and init.grad.shape == init.shape
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("channel_last", [False, True], ids=["cf", "cl"])
 @pytest.mark.parametrize("extra", ["none", "states", "seq_idx", "no_bias"])
