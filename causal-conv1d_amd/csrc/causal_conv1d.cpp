@@ -13,6 +13,7 @@
 #include <torch/library.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <ATen/PythonTorchFunctionTLS.h>
@@ -626,8 +627,35 @@ variable_list recorded(const at::Tensor &x, const at::Tensor &weight, const std:
                        const std::optional<at::Tensor> &seq_idx, const std::optional<at::Tensor> &init) {
     return CausalConv1dFn<HOW>::apply(x, weight, bias, seq_idx, init);
 }
-constexpr decltype(&recorded<0>) recorders[] = {recorded<0>, recorded<1>, recorded<2>, recorded<3>,
-                                                recorded<4>, recorded<5>, recorded<6>, recorded<7>};
+constexpr variable_list (*recorders[])(const at::Tensor &, const at::Tensor &, const std::optional<at::Tensor> &,
+                                       const std::optional<at::Tensor> &, const std::optional<at::Tensor> &) = {
+    recorded<0>, recorded<1>, recorded<2>, recorded<3>,
+    recorded<4>, recorded<5>, recorded<6>, recorded<7>};
+
+// A node's Python object: what every C++ node's has, and saved_tensors, as on the Python function's.
+template <int HOW>
+PyObject *saved_tensors(PyObject *self, void *) {
+    HANDLE_TH_ERRORS
+    using Node = torch::autograd::CppNode<CausalConv1dFn<HOW>>;
+    variable_list saved = static_cast<Node *>(reinterpret_cast<torch::autograd::THPCppFunction *>(self)->cdata.get())->ctx_.get_saved_variables();
+    PyObject *all = PyTuple_New((Py_ssize_t)saved.size());
+    if (all == nullptr) throw python_error();
+    for (size_t i = 0; i < saved.size(); ++i) PyTuple_SET_ITEM(all, (Py_ssize_t)i, THPVariable_Wrap(std::move(saved[i])));
+    return all;
+    END_HANDLE_TH_ERRORS
+}
+template <int HOW>
+void register_node() {
+    using namespace torch::autograd;                  // the names in the macro
+    static PyTypeObject type = {};
+    static PyGetSetDef properties[] = {THP_FUNCTION_DEFAULT_PROPERTIES,
+                                       {"saved_tensors", &saved_tensors<HOW>, nullptr, nullptr, nullptr},
+                                       {nullptr, nullptr, nullptr, nullptr, nullptr}};
+    registerCppFunction(typeid(CppNode<CausalConv1dFn<HOW>>), _initFunctionPyTypeObject(type, "CausalConv1dFnBackward", properties, nullptr));
+}
+template <int... HOW>
+void register_nodes(std::integer_sequence<int, HOW...>) { (register_node<HOW>(), ...); }
+
 // What only the Python function answers for: functorch transforms and forward-mode gradients, which it refuses in its own words.
 bool python_graph_needed(const std::optional<at::Tensor> &t) { return t.has_value() && (t->has_names() || t->_fw_grad(0).defined()); }
 
@@ -722,6 +750,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("causal_conv1d_varlen_states", &causal_conv1d_varlen_states, "Varlen final-state gather");
     m.def("causal_conv1d_fwd_varlen_states", &causal_conv1d_fwd_varlen_states,
           "Causal conv1d forward and varlen final-state gather in one call");
+    register_nodes(std::make_integer_sequence<int, (int)std::size(recorders)>{});
     if (PyModule_AddFunctions(m.ptr(), direct_calls) != 0) throw pybind11::error_already_set();
 }
 

@@ -110,6 +110,28 @@ def test_every_gradient_arrives(pkg, monkeypatch, between, compiled):
     assert native == python == ([(2, 8, 9), (8, 4), (8,), (2, 8, 3)],) * 2
 
 
+def test_saved_tensors_of_the_node(pkg, monkeypatch):
+    """On meta tensors, without a GPU: grad_fn.saved_tensors in every combination of activation, final states and states."""
+    def run():
+        seen = []
+        for activation in (None, "silu"):
+            for final in (False, True):
+                for init in (None, _meta(2, 8, 3), _meta(2, 8, 3, grad=True)):
+                    x, w = _meta(2, 8, 9, grad=True), _meta(8, 4)
+                    out = pkg.causal_conv1d_fn(x, w, initial_states=init, return_final_states=final, activation=activation)
+                    out = out[0] if final else out
+                    saved = out.grad_fn.saved_tensors
+                    assert len(saved) == 5 and saved[0] is x and saved[1] is w and saved[4] is init
+                    seen.append((type(out.grad_fn).__name__, [t if t is None else tuple(t.shape) for t in saved]))
+                    out.sum().backward()
+                    with pytest.raises(RuntimeError, match="second time"):
+                        out.grad_fn.saved_tensors
+        return seen
+
+    native, python = _both(monkeypatch, run)
+    assert native == python
+
+
 def test_gradient_of_states_that_need_a_copy(pkg):
     """On meta tensors, without a GPU: initial_states with no unit stride are copied first, and keep their gradient."""
     x, w, init = _meta(2, 8, 9, grad=True), _meta(8, 4), _meta(2, 16, 6, grad=True)
