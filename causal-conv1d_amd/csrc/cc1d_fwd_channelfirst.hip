@@ -16,7 +16,7 @@
 // initial_states / final_states are supported (the reference refuses them for this
 // layout, csrc/causal_conv1d.cpp:213,228).
 //
-// Three kernels share this design.  The streaming kernel takes every launch in which the rows
+// Four kernels share this design.  The streaming kernel takes every launch in which the rows
 // of out lie on the same 16-byte grid as the rows of x (same shape and strides, as
 // empty_like gives): whole 64-vector steps run without bounds checks in two register sets in
 // ping-pong, which keep the loads of the next two groups in flight while a group is computed
@@ -25,7 +25,8 @@
 // three steps start their steps on 128-byte lines of out, with a partly filled first step; and
 // the few positions of a row in front of its first whole vector or behind its last one are
 // produced one per lane, straight from memory.  The general kernel takes out tensors on a different grid.  The short-row
-// kernel takes rows of at most 64 vectors, several rows to a wavefront and no walk.  Rows of
+// kernel takes rows of at most 64 vectors, several rows to a wavefront and no walk; the flat kernel
+// takes such rows of a contiguous tensor as whole vectors of one flat array where that is faster.  Rows of
 // more than 64 vectors that start on 128-byte lines (tensors of up to 512 MiB) or hold at most
 // 128 vectors, and rows off the 16-byte grid of up to 512 vectors (192 of fp32), go to the tile
 // kernel of cc1d_fwd_channelfirst_tile.hip (rows fetched straight into LDS; 1-25 % faster on
@@ -590,6 +591,207 @@ int launch_short(const cc1d_fwd_params &p, int n_vecs, bool aligned, hipStream_t
     return launch_status();
 }
 
+// Short rows of a contiguous tensor whose seqlen is no multiple of the vector length (at least
+// one vector, at most 64), where flat_is_faster says so: rows then start anywhere on the 16-byte grid, but batch * dim * seqlen
+// elements lie back to back, so a lane owns one whole vector of that flat array: one 16-byte load
+// and one 16-byte store, and no lane is without a vector; the short-row kernel has fewer instructions to a
+// lane, but idle lanes, and vectors that straddle the grid.
+// A vector spans at most two rows; the lane holds the taps of both, takes its left neighbours from
+// the previous lane (lane 0 of a wavefront from memory) and masks the taps that reach in front of
+// a row's start (or takes initial_states there).  Same arithmetic, in the same order, as the
+// other kernels.
+template <int DT, int W, bool SILU, bool PACKED_W>
+__global__ void __launch_bounds__(kBlock)
+fwd_channelfirst_flat_kernel(const cc1d_fwd_params p, const uint32_t n_elems) {
+    using E = Elem<DT>;
+    using T = typename E::type;
+    constexpr int VEC = E::kVec;
+    constexpr bool PRECISE = E::kPreciseAct;
+    constexpr bool SCALED = SILU && !PRECISE;
+
+    const uint32_t gid = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t L = (uint32_t)p.seqlen, D = (uint32_t)p.dim;
+    // Lanes past the end stay in step (the lane shift needs every lane) on vector 0.
+    const bool mine = (uint64_t)gid * VEC < n_elems;
+    const uint32_t f0 = mine ? gid * VEC : 0u;
+    const bool whole = f0 + VEC <= n_elems;           // only the array's last vector can be partial
+
+    u32x4 raw = u32x4{0u, 0u, 0u, 0u};
+    if (mine) {
+        if (whole) {
+            raw = ld_vec_nt<DT>(p.x, f0);
+        } else {
+            T elems[VEC];
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) elems[e] = f0 + e < n_elems ? ld_raw<DT>(p.x, f0 + e) : T(0.f);
+            __builtin_memcpy(&raw, elems, sizeof raw);
+        }
+    }
+    const uint32_t row0 = f0 / L;
+    const uint32_t t0 = f0 - row0 * L;
+    const uint32_t split = L - t0;                    // elements [split, VEC) belong to the next row
+    const uint32_t c0 = row0 % D, b0 = row0 / D;
+    const bool wrap = c0 + 1 == D;
+    const uint32_t c1 = wrap ? 0u : c0 + 1, b1 = wrap ? b0 + 1 : b0;
+
+    // Taps of the row the vector starts in, and of the next one only where the vector reaches it
+    // (one lane in seqlen / VEC).  Packed fp32 taps (a host-checked promise: strides (W, 1), base
+    // 16-byte aligned) of even width come in one load.
+    float w0[W], w1[W], bias0, bias1 = 0.f;
+    auto taps = [&](uint32_t c, float (&wv)[W], float &bv) {
+        if (PACKED_W && W % 2 == 0) {
+            const float *src = static_cast<const float *>(__builtin_assume_aligned(
+                reinterpret_cast<const float *>(p.weight) + (int64_t)c * W, W % 2 == 0 ? W * 4 : 4));
+#pragma unroll
+            for (int w = 0; w < W; ++w) wv[w] = src[w];
+            bv = p.bias == nullptr ? 0.f : reinterpret_cast<const float *>(p.bias)[c];   // of the taps' type
+        } else {
+            channel_taps<W>(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, (int)c, wv, bv);
+        }
+    };
+    taps(c0, w0, bias0);
+#pragma unroll
+    for (int w = 0; w < W; ++w) w1[w] = 0.f;
+    if (split < (uint32_t)VEC) taps(c1, w1, bias1);
+    if (SCALED) {
+        bias0 *= kSiluPrescale;
+        bias1 *= kSiluPrescale;
+#pragma unroll
+        for (int w = 0; w < W; ++w) { w0[w] *= kSiluPrescale; w1[w] *= kSiluPrescale; }
+    }
+
+    float xf[VEC];
+    E::unpack(raw, xf);
+    // xx[i] = flat element f0-(W-1)+i
+    float xx[VEC + W - 1];
+    float first[W - 1];
+#pragma unroll
+    for (int i = 0; i < W - 1; ++i) first[i] = 0.f;
+    if (lane == 0 && f0 >= (uint32_t)(W - 1)) {
+#pragma unroll
+        for (int i = 0; i < W - 1; ++i) first[i] = ld_elem<DT>(p.x, (int64_t)f0 - (W - 1) + i);
+    }
+#pragma unroll
+    for (int i = 0; i < W - 1; ++i) xx[i] = from_prev_lane(xf[VEC - (W - 1) + i], first[i]);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) xx[W - 1 + e] = xf[e];
+
+    const bool has_init = p.initial_states != nullptr;
+    float acc[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+        const bool next = (uint32_t)e >= split;
+        const uint32_t t = next ? (uint32_t)e - split : t0 + (uint32_t)e;
+        float a = next ? bias1 : bias0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            // tap w reads position t-(W-1-w) of the row
+            float xv = xx[e + w];
+            if (w < W - 1 && t + (uint32_t)w < (uint32_t)(W - 1)) {
+                xv = 0.f;
+                if (has_init && f0 + e < n_elems)     // (positions past the array's end belong to no row)
+                    xv = ld_elem<DT>(p.initial_states, (int64_t)(next ? b1 : b0) * p.init_stride_b +
+                                                           (int64_t)(next ? c1 : c0) * p.init_stride_c +
+                                                           (int64_t)(t + w) * p.init_stride_l);
+            }
+            a = fmaf(next ? w1[w] : w0[w], xv, a);
+        }
+        acc[e] = SCALED ? silu_from_scaled(a) : SILU ? silu<PRECISE>(a) : a;
+    }
+    if (mine) {
+        if (whole) {
+            st_vec_nt<DT>(p.out, f0, E::pack(acc));
+        } else {
+#pragma unroll
+            for (int e = 0; e < VEC; ++e)
+                if (f0 + e < n_elems) st_elem<DT>(p.out, f0 + e, acc[e]);
+        }
+    }
+
+    // final_states[b, c, i] = x[L-(W-1)+i] (a row is never shorter than a vector, so never
+    // shorter than W-1), bit-exact copies, by the lane whose vector holds the row's last element.
+    if (p.final_states != nullptr && mine && split <= (uint32_t)VEC && f0 + split <= n_elems) {
+#pragma unroll
+        for (int i = 0; i < W - 1; ++i) {
+            const T e = ld_raw<DT>(p.x, (int64_t)f0 + split - (W - 1) + i);
+            st_raw<DT>(p.final_states, (int64_t)b0 * p.final_stride_b + (int64_t)c0 * p.final_stride_c +
+                                           (int64_t)i * p.final_stride_l, e);
+        }
+    }
+}
+
+// Where the flat kernel is the faster of the two.  It takes the instructions of two rows' taps to a vector, and
+// with initial_states a branch to every tap; the short-row kernel idle lanes (a row takes a power of two of them),
+// vectors that straddle the grid and a last one in pieces.  So the flat array wins where little is computed (no
+// activation, narrow taps), where few of the lanes have work, and where its wavefronts fit the chip at once while
+// the other kernel's do not.  Rows of a multiple of four vectors, and 16-bit rows of even length, straddle less.
+// us flat / short, width 4 and SiLU: bf16 (27, 4096, 9) 4.6 / 4.1, (1085, 4096, 9) 51.7 / 64.8, (976, 4096, 10) 51.2 / 41.0,
+// (295, 4096, 33) 51.0 / 60.7, (325, 4096, 30) 51.2 / 35.8, (16, 5376, 100) 15.0 / 11.1, (37, 4096, 257) 50.4 / 46.2, fp32
+// (147, 4096, 33) 40.7 / 51.6, (376, 4096, 13) 41.0 / 32.6, (8, 2048, 250) 10.6 / 9.5; without SiLU bf16 (256, 4096, 9) 12.3 / 17.8,
+// fp32 (64, 4096, 33) 15.4 / 24.1; width 2 bf16 (256, 4096, 9) 12.6 / 14.4; width 3 bf16 (256, 4096, 23) 27.9 / 35.8, fp32
+// (64, 4096, 65) 27.2 / 35.3.  12000 calls over types, widths, activation, states, lengths and 1500 .. 140000
+// wavefronts: flat throughout 1, short throughout 0.948 (a third of them 3 % slower and more, up to 90 %), by this
+// rule 0.914 (1.4 % of them, up to 21 %), the faster of the two each time 0.906.
+bool flat_is_faster(const cc1d_fwd_params &p, int64_t vecs, int vec) {
+    constexpr int64_t kChip = 8192;                   // wavefronts: 32 on each of 256 CUs
+    constexpr int kAlways = 101;
+    int64_t lanes = 1;
+    while (lanes < vecs) lanes *= 2;
+    const int64_t rows = (int64_t)p.batch * p.dim;
+    const int64_t waves = rows * lanes / kWave, flat_waves = rows * p.seqlen / (vec * kWave);
+    const bool silu = p.silu != 0, w2 = p.width == 2, heavy = p.width == 4 && silu;
+    const bool init = p.initial_states != nullptr, final = p.final_states != nullptr;
+    const bool is32 = p.x_dtype == CC1D_F32, quads = vecs % 4 == 0, rough = p.seqlen % 2 != 0 && !quads;
+    // The percentage of the lanes' positions that rows fill below which the flat array wins.
+    int below;
+    if (is32) {
+        if (heavy) below = quads ? 0 : init ? 57 : final ? 80 : 72;
+        else if (init) below = silu ? 60 : 86;
+        else if (final && quads) below = 70;
+        else below = w2 && silu ? (final ? 60 : 75) : kAlways;
+    } else if (init) {
+        below = w2 ? 60 : 0;
+    } else if (w2 && (rough || !silu)) {
+        below = final && !rough ? 66 : kAlways;
+    } else if (rough) {
+        below = vecs > 16 ? (heavy ? 0 : 60) : heavy ? 74 : silu ? 80 : 97;
+    } else if (final) {
+        below = !silu ? 72 : quads ? 0 : 60;
+    } else {
+        below = w2 ? 70 : silu || quads ? 0 : 60;
+    }
+    if (below == kAlways) return true;
+    const int64_t filled = p.seqlen * 100 / (lanes * vec);
+    const bool one_round = flat_waves <= kChip && waves > (heavy || (!is32 && !w2) ? kChip : kChip / 2);
+    if (below == 0) return one_round && filled < 70 && (is32 || (!heavy && !init));
+    return one_round || (waves > (heavy && !is32 ? kChip : kChip / 2) && filled < below);
+}
+
+template <int DT>
+int launch_flat(const cc1d_fwd_params &p, hipStream_t stream) {
+    constexpr int VEC = Elem<DT>::kVec;
+    const uint32_t n_elems = (uint32_t)((int64_t)p.batch * p.dim * p.seqlen);
+    const uint32_t n_vecs = (n_elems + VEC - 1) / VEC;
+    const dim3 grid((n_vecs + kBlock - 1) / kBlock), block(kBlock);
+    const bool packed = weights_contiguous_f32(p.weight, p.w_dtype, p.w_stride_c, p.w_stride_w, p.width);
+#define CC1D_FLAT2(WIDTH, SILU_ON)                                                                                    \
+    if (packed) CC1D_LAUNCH((fwd_channelfirst_flat_kernel<DT, WIDTH, SILU_ON, true>), grid, block, 0, stream,  \
+                                   p, n_elems);                                                                       \
+    else CC1D_LAUNCH((fwd_channelfirst_flat_kernel<DT, WIDTH, SILU_ON, false>), grid, block, 0, stream, p,     \
+                            n_elems)
+#define CC1D_FLAT(WIDTH)                                                                                              \
+    if (p.silu) { CC1D_FLAT2(WIDTH, true); } else { CC1D_FLAT2(WIDTH, false); }
+    switch (p.width) {
+        case 2: CC1D_FLAT(2); break;
+        case 3: CC1D_FLAT(3); break;
+        default: CC1D_FLAT(4); break;
+    }
+#undef CC1D_FLAT
+#undef CC1D_FLAT2
+    return launch_status();
+}
+
 template <int DT, bool SILU, int U, bool BI>
 int launch_stream(const cc1d_fwd_params &p, const FwdCfGeom &g, hipStream_t stream) {
     const uint32_t blocks = (g.total_waves + (kBlock / kWave) - 1) / (kBlock / kWave);
@@ -647,16 +849,31 @@ int launch_fwd_channelfirst(const cc1d_fwd_params &p, hipStream_t stream) {
     // Short rows of whole vectors, up to eight to a wavefront, no walk: (4, 5376, 256) bf16 11.2 -> 6.0 us,
     // (8, 1024, 512) bf16 6.7 -> 4.8 us, (4, 5376, 256) fp32 10.9 -> 8.5 us, (1, 5376, 64) bf16 4.8 -> 3.3 us.
     // Rows that are not whole vectors on one grid take the same lanes, vectors of any address and the last one of
-    // a row in pieces, or single elements where a row is shorter than a vector.  Against whole vectors of the flat
-    // array, each with the taps of the two rows it may span (contiguous tensors; others took elements):
-    // (8, 4096, 500) bf16 22.6 -> 14.8 us, (16, 5376, 100) 14.8 -> 10.8, (64, 2048, 60) 12.8 -> 9.0, (4, 1024, 300) 5.1 -> 3.4,
-    // (32, 4096, 250) 42.9 -> 25.6, (8, 2048, 250) fp32 10.4 -> 9.0, and where half of the lanes have no vector
-    // (16, 2048, 265) 15.4 -> 14.0, (16, 5376, 130) 17.2 -> 16.0; (3, 6000, 77) with states 7.4 -> 5.0.
-    // (256, 5376, 4) 360 -> 11.9 us walking -> elements.
+    // a row in pieces, or single elements where a row is shorter than a vector: against elements throughout
+    // (16, 5376, 100) bf16 25.4 -> 10.8 us, (64, 2048, 60) 16.4 -> 9.0; (256, 5376, 4) 360 -> 11.9 us walking -> elements.
     const int64_t short_vecs = ((int64_t)p.seqlen + vec - 1) / vec;
     const int32_t forced_vecs = tunables().fwd_cf_vecs;
     if (short_vecs <= 64 && forced_vecs <= 0) {
         const bool aligned = same_grid && on_grid && p.seqlen % vec == 0;
+        // A contiguous tensor of rows that are not whole vectors, but at least one: the flat array, or the lanes of
+        // the short rows all the same.
+        const int64_t n_elems = rows * p.seqlen;
+        // (Not when final_states may be the buffer initial_states come from: in the flat walk the
+        // lane that reads a row's initial_states and the lane that writes its final_states can sit in
+        // different wavefronts.)
+        const bool states_in_and_out = p.initial_states != nullptr && p.final_states != nullptr;
+        const bool flat = !aligned && !states_in_and_out && p.seqlen >= vec && n_elems < thread_limit() &&
+                          aligned16(p.x) && aligned16(p.out) &&
+                          (p.dim == 1 || (p.x_stride_c == p.seqlen && p.out_stride_c == p.seqlen)) &&
+                          (p.batch == 1 || (p.x_stride_b == (int64_t)p.dim * p.seqlen &&
+                                            p.out_stride_b == (int64_t)p.dim * p.seqlen));
+        if (flat && flat_is_faster(p, short_vecs, vec)) {
+            switch (p.x_dtype) {
+                case CC1D_F32: return launch_flat<CC1D_F32>(p, stream);
+                case CC1D_F16: return launch_flat<CC1D_F16>(p, stream);
+                default: return launch_flat<CC1D_BF16>(p, stream);
+            }
+        }
         switch (p.x_dtype) {
             case CC1D_F32: return launch_short<CC1D_F32>(p, (int)short_vecs, aligned, stream);
             case CC1D_F16: return launch_short<CC1D_F16>(p, (int)short_vecs, aligned, stream);
