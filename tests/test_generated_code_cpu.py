@@ -1,0 +1,33 @@
+"""What the compiler makes of kernels whose speed turns on it, read from their gfx950 assembly; needs no GPU."""
+import os
+import re
+import subprocess
+import sys
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, os.path.join(ROOT, "causal-conv1d_amd"))
+
+
+def _assembly(source, tmp_path):
+    import build
+    path = str(tmp_path / (source + ".s"))
+    cmd = build.compile_command(source, path, ["--cuda-device-only", "-S"])
+    cmd.remove("-c")
+    subprocess.run(cmd, check=True, capture_output=True, timeout=300)
+    return open(path).read()
+
+
+def _kernels(text, name):
+    """(mangled name, body) of every instance of a kernel."""
+    found = re.findall(r"^(_ZN\S*%s\S+):.*?\n(.*?)^\.Lfunc_end" % name, text, re.S | re.M)
+    assert found
+    return found
+
+
+def test_backward_tiles_do_not_wait_for_their_stores(tmp_path):
+    """Behind the first store of dx nothing is left to wait for but stores: a vector-memory wait there holds a step up
+    until the one in front has been written.  (A workgroup that adds up its own sums may add into memory at the end.)"""
+    for name, body in _kernels(_assembly("cc1d_bwd_channelfirst_tile.hip", tmp_path), "bwd_channelfirst_tile_kernel"):
+        steps = body[body.index("buffer_store_dwordx4"):]
+        direct = re.search(r"tile_kernelILi\dELi\dELb[01]ELb([01])E", name).group(1) == "1"
+        assert steps.count("s_waitcnt vmcnt") <= direct, name
