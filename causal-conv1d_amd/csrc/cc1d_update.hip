@@ -439,14 +439,20 @@ update_tokens_kernel(const TokensArgs ta) {
     Staging staging;
     staging.request(a.weight, a.bias, col0, cols_here);
 
-    // As in the step kernel: the x rows wait for nothing, the state rows for the slot and the position.
+    // As in the step kernel: the x rows wait for nothing, the state rows for the slot and the position.  The x rows
+    // are asked for in a function of their own: as statements of the kernel the compiler holds all eight rows together
+    // and copies them at every branch, in 128 to 150 registers instead of 62, with a wait behind every load.  500
+    // calls of 2 .. 8 tokens over types, widths, rings and slots: 27 % less on average (8 tokens 40 %), none slower;
+    // bf16 ring (256, 584, 5 tokens) in slots 6.5 -> 4.4 us.
     int cs = CIRC ? a.cache_seqlens[b] : 0;
     raw_t rw[W - 1], xr[kMaxTokens];
+    [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kMaxTokens; ++i) {
-        xr[i] = P::zero();
-        if (i < L) xr[i] = *reinterpret_cast<const raw_t *>(xrow + (int64_t)i * ta.x_stride_l);
-    }
+        for (int i = 0; i < kMaxTokens; ++i) {
+            xr[i] = P::zero();
+            if (i < L) xr[i] = *reinterpret_cast<const raw_t *>(xrow + (int64_t)i * ta.x_stride_l);
+        }
+    }();
     const int srow = a.conv_state_indices == nullptr ? b : a.conv_state_indices[b];
     T *st = reinterpret_cast<T *>(a.conv_state) + (int64_t)(srow < 0 ? 0 : srow) * a.state_stride_b + c0;
     int first = S - (W - 1);

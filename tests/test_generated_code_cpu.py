@@ -31,3 +31,10 @@ def test_backward_tiles_do_not_wait_for_their_stores(tmp_path):
         steps = body[body.index("buffer_store_dwordx4"):]
         direct = re.search(r"tile_kernelILi\dELi\dELb[01]ELb([01])E", name).group(1) == "1"
         assert steps.count("s_waitcnt vmcnt") <= direct, name
+
+
+def test_decode_of_a_few_tokens_keeps_eight_waves(tmp_path):
+    """At most 64 registers, eight wavefronts a SIMD, with up to eight x rows in flight."""
+    text = _assembly("cc1d_update.hip", tmp_path)
+    counts = re.findall(r"\.name:\s+\S*update_tokens_kernel\S*.*?\.vgpr_count:\s+(\d+)", text, re.S)
+    assert counts and all(int(n) <= 64 for n in counts), counts
