@@ -767,19 +767,21 @@ bool rows_lane_ok(const void *ptr, int dtype, int lane_bytes, int64_t sb, int64_
 constexpr int kStepLaneBytes = 8;
 constexpr int kStepRowsMax = 2;                    // batch rows per lane: one or two
 
-// One, except in a launch that two rows a lane bring to just under two workgroups for each of the 256 CUs: one
-// row a lane would then be just under four, twice the workgroups for the same evenness.  Everywhere else one row
-// has the shorter chain and twice the wavefronts in flight.  us a launch over 40 rotating sets, two rows / one row
-// (workgroups with two rows): bf16 batch 8, dim 5376, state 4 (21) 2.72 / 2.42; 32 (84) 2.96 / 2.73; (128, 5376, 3) (336)
-// 4.11 / 3.69; (256, 2560, 3) (320) 4.09 / 3.68; fp32 (64, 5376, 4) in 128 slots (336) 4.24 / 3.85; (224, 5376, 3) (588)
-// 5.44 / 5.26; (256, 5376, 3) (672) 5.74 / 5.75; (512, 2560, 3) (640) 5.63 / 5.69; (512, 5376, 4) (1344) 10.85 / 10.56;
-// (1024, 5376, 3) (2688) 16.79 / 16.51; and kept at two, ring fp16 (384, 2560, 8) (480) 4.12 / 4.17, (192, 5376, 4) (504)
-// 4.89 / 5.06, fp32 (96, 5376, 3) (504) 4.38 / 4.56, (256, 4096, 3) (512) 4.50 / 4.55.  Three and four rows are
-// slower at every size.
-bool two_step_rows(int64_t column_blocks, int64_t batch) {
+// One, except in a launch that two rows a lane bring to just under two or three workgroups for each of the 256 CUs: one
+// row a lane would then be just under four or six, twice the workgroups for the same evenness.  Elsewhere one row
+// has the shorter chain and more wavefronts in flight; so it has with two rows and more in front of the window, which a
+// lane shifts one after the other.  Time with two rows / with one over 900 calls of every type and width, 400 .. 1500
+// workgroups with two rows, 24 rotating sets: rings 1.00 at 400 .. 431, 0.99 at 432 .. 448, 0.984 at 449 .. 512, 1.01 .. 1.03 at
+// 513 .. 656, 0.982 at 657 .. 768, 1.01 above; states as long as the window 1.01 up to 656, 0.976 at 657 .. 768, 1.02 above; one row
+// in front of it 0.990, 1.03, 1.00; two and more 1.13 .. 1.26 up to 768, 1.08 at 897 .. 1024.  us, two rows / one
+// (workgroups with two rows): bf16 batch 8, dim 5376, state 4 (21) 2.72 / 2.42; (128, 5376, 3) (336) 4.11 / 3.69; ring fp16
+// (384, 2560, 8) (480) 4.12 / 4.17, (192, 5376, 4) (504) 4.89 / 5.06; fp32 (224, 5376, 3) (588) 5.44 / 5.26; fp16 (514, 2584, 3) in slots
+// (715) 7.18 / 7.43; bf16 (512, 5376, 4) (1344) 10.85 / 10.56.  Three and four rows are slower at every size.
+bool two_step_rows(int64_t column_blocks, int64_t batch, int rows_shifted) {
     const int64_t two = column_blocks * ((batch + 2 * kStepWaves - 1) / (2 * kStepWaves));
     const int64_t one = column_blocks * ((batch + kStepWaves - 1) / kStepWaves);
-    return (two > 448 && two <= 512) || one * kBlock >= thread_limit();
+    const bool even = (two > 448 && two <= 512) || (two > 656 && two <= 768);
+    return (even && rows_shifted < 2) || one * kBlock >= thread_limit();
 }
 
 template <int DT, int W>
@@ -804,7 +806,7 @@ int launch_w(const cc1d_update_params &p, bool vec, hipStream_t stream) {
         a.batch = p.batch; a.state_len = p.state_len;
         a.n_colgroups = (uint32_t)(p.dim / CH);
         const uint32_t column_blocks = (a.n_colgroups + kWave - 1) / kWave;
-        const bool two_rows = two_step_rows(column_blocks, p.batch);
+        const bool two_rows = two_step_rows(column_blocks, p.batch, circ ? 0 : p.state_len - (W - 1));
         const int block_rows = kStepWaves * (two_rows ? 2 : 1);
         const dim3 grid(column_blocks, (uint32_t)((p.batch + block_rows - 1) / block_rows));
         if ((int64_t)grid.x * grid.y * kBlock >= thread_limit()) return CC1D_ERR_TOO_LARGE;

@@ -1,6 +1,6 @@
 """The decode step with one and with two batch rows a lane: batches at the edges of the rule that chooses (two
-rows where they come to 449 .. 512 workgroups of eight batch rows and 64 column groups each), and batches
-that are no whole number of a workgroup's rows.  Outputs against the plain PyTorch step, the cache bit for bit."""
+rows where they come to 449 .. 512 or 657 .. 768 workgroups of eight batch rows and 64 column groups each and at
+most one row lies in front of the window), and batches that are no whole number of a workgroup's rows.  Outputs against the plain PyTorch step, the cache bit for bit."""
 import pytest
 import torch
 
@@ -15,9 +15,18 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("ring", [False, True], ids=["shift", "ring"])
 @pytest.mark.parametrize("blocks,batch", [(1, 1), (3, 5), (1, 3584), (1, 3585), (1, 4093), (1, 4096), (1, 4097), (7, 511), (7, 513), (8, 505)])
 def test_step_rows(pkg, gpu_device, blocks, batch, ring, dtype):
+    _check(pkg, gpu_device, blocks, batch, ring, dtype, 8 if ring else 3)
+
+
+@pytest.mark.parametrize("ring", [False, True], ids=["shift", "ring"])
+@pytest.mark.parametrize("blocks,batch,state_len", [(1, 5248, 3), (1, 5249, 4), (3, 1755, 5), (3, 2041, 4), (1, 6144, 3), (1, 6145, 3), (1, 3585, 4), (1, 4096, 5)])
+def test_step_rows_in_front_of_the_window(pkg, gpu_device, blocks, batch, ring, state_len):
+    _check(pkg, gpu_device, blocks, batch, ring, torch.bfloat16, state_len)
+
+
+def _check(pkg, gpu_device, blocks, batch, ring, dtype, state_len):
     g = gen(10 * batch + blocks)
     D = blocks * 64 * (8 // torch.empty(0, dtype=dtype).element_size()) - 8      # the last block a partial one
-    state_len = 8 if ring else 3
     state = torch.randn(batch, state_len, D, generator=g).to(dtype).transpose(1, 2)
     x = torch.randn(batch, 1, D, generator=g).to(dtype).transpose(1, 2)
     w, b = make_wb(D, 4, True, g)
