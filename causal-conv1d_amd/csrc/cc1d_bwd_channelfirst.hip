@@ -27,9 +27,10 @@
 // partly filled last step of a row are done first, one checked step at a time, and the few
 // positions of a row in front of its first whole vector or behind its last one are done one
 // per lane, straight from memory.  The general kernel takes tensors on different grids and
-// rows longer than 64 vectors.  The short-row kernel takes rows of at most 64 vectors (whole
-// vectors on one grid, or element by element), several batch entries of a channel to a
-// wavefront and no walk.
+// rows longer than 64 vectors.  The short-row kernel takes rows of at most 64 vectors, several
+// batch entries of a channel to a wavefront and no walk: whole vectors on one grid (kWhole), vectors
+// of any address with the last one of a row in pieces (kAnywhere), or, for rows shorter than a
+// vector, single elements (kElements).
 //
 // Rows longer than 64 vectors normally do not reach these walking kernels: the tile kernel of
 // cc1d_bwd_channelfirst_tile.hip takes them (a wavefront per tile of up to 256 vectors of one
@@ -960,18 +961,20 @@ BwdCfGeom make_geom(const cc1d_bwd_params &p) {
 // Short rows whose kernel adds up a channel's parts itself (see DIRECT).  What the second launch costs
 // stays the same, what the other form costs grows with the launch:
 //  * A workgroup's wavefronts must find room on one CU together and hold it until the last of them ends.  The
-//    kernels take 49-75 registers, and 80-93 for 16-bit rows off the vector grid, five to eight wavefronts a
-//    SIMD; 13 to 16 to a workgroup then leave up to half of the slots empty, 9 to 12 and 5 to 8 fewer.  So
-//    large workgroups only where each has a CU of its own (256 channels) or enough of them fit, and few items
-//    to a wavefront, one after the other.
+//    kernels take 49 to 81 registers, six to eight wavefronts a SIMD; 13 to 16 to a workgroup then leave up to
+//    half of the slots empty, smaller ones less.  So those only where each has a CU of its own (256 channels), and
+//    few items to a wavefront, one after the other.
 //  * Channels whose rows share cache lines go to different XCDs, where two or three parts leave room for another
 //    channel in a workgroup of four.  So two items at most there, and next to nothing of rows of a few dwords.
-// Two launches / one, us, parts x items: (4, 1024, 300) bf16 4 x 1 11.3 / 8.7, (32, 256, 64) 4 x 1 6.5 / 4.3,
-// (8, 512, 512) 8 x 1 8.4 / 6.0, (8, 2048, 512) 2 x 4 15.6 / 12.7, (80, 410, 64) 10 x 1 8.3 / 6.4, (16, 256, 509) 16 x 1
-// 13.0 / 10.8, but (14, 300, 512) 14 x 1 8.6 / 9.1, (16, 64, 509) 8.1 / 8.8, (18, 818, 512) 6 x 3 13.8 / 14.3,
-// (32, 4095, 61) 2 x 2 39.1 / 40.1, (96, 683, 509) 6 x 16 131 / 195, (224, 300, 512) 14 x 16 48.9 / 67.1,
-// (256, 256, 512) 16 x 16 41.7 / 45.3, and for the lines (240, 2048, 16) 2 x 4 32.9 / 44.9, (124, 2048, 48) 2 x 8 28.0 / 36.1,
-// (992, 64, 8) 16 x 1 8.4 / 14.7.
+//  * 16-bit rows off the vector grid and fp32 ones keep lines of their own, narrower than their kernel now needs
+//    (they were drawn when it took 80 to 93 registers): 500 launches between them and those of rows on the grid
+//    ran 0.72 to 1.02 of the time of two launches, 0.84 on average, on cold buffers.
+// Two launches / one, us bf16, parts x items: (4, 1024, 300) 4 x 1 8.8 / 6.7, (32, 256, 64) 4 x 1 5.7 / 3.9, (8, 512, 512) 8 x 1
+// 7.6 / 5.7, (8, 2048, 512) 2 x 4 16.6 / 12.6, (80, 410, 64) 10 x 1 7.5 / 5.9, (16, 256, 509) 16 x 1 10.1 / 7.7;
+// not taken (100, 700, 100) 5 x 5 20.4 / 18.1, (14, 300, 512) 14 x 1 8.2 / 8.0, (14, 300, 509) 10.7 / 11.7, (18, 818, 512) 6 x 3 14.0 / 12.2,
+// (18, 818, 509) 18.0 / 18.2, (32, 4095, 61) 2 x 2 21.3 / 20.3, (16, 64, 509) 16 x 1 6.7 / 6.4, (96, 683, 509) 6 x 16 54.2 / 53.4,
+// (224, 300, 512) 14 x 16 48.6 / 68.1, (256, 256, 512) 16 x 16 41.8 / 50.0, and for the lines (240, 2048, 16) 2 x 4 32.8 / 44.5,
+// (124, 2048, 48) 2 x 8 27.5 / 35.9, (992, 64, 8) 16 x 1 8.1 / 14.6.
 bool short_rows_direct(const cc1d_bwd_params &p, const BwdCfGeom &g) {
     if ((g.streaming != 3 && g.streaming != 4) || g.n_parts <= 1 || tunables().bwd_cf_direct < 0) return false;
     constexpr int kCus = 256, kLine = 128;
