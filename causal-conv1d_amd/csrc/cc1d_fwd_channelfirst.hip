@@ -479,15 +479,17 @@ fwd_channelfirst_short_kernel(const cc1d_fwd_params p, const int n_vecs, const i
     } else if (ROWS == kAnywhere) {
         if (mine) raw = ld_vec_any<DT>(p.x, xrow + v * VEC - shared / E::kBytes);
     } else {
-        T elems[VEC];
+        // In a function of its own: as statements of the kernel the compiler waits for the first element (16-bit: for
+        // each) in front of the next one's request: fp32 (686, 3358, 2) 17.3 -> 15.9 us, bf16 (57, 1714, 5) 3.48 -> 3.23.
+        [&]() __attribute__((always_inline)) {
+            T elems[VEC];
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) elems[e] = T(0.f);
-        if (mine) {
-#pragma unroll
-            for (int e = 0; e < VEC; ++e)
-                if (v * VEC + e < L) elems[e] = ld_raw<DT>(p.x, xrow + v * VEC + e);
-        }
-        __builtin_memcpy(&raw, elems, sizeof raw);
+            for (int e = 0; e < VEC; ++e) {
+                elems[e] = T(0.f);
+                if (mine && v * VEC + e < L) elems[e] = ld_raw<DT>(p.x, xrow + v * VEC + e);
+            }
+            __builtin_memcpy(&raw, elems, sizeof raw);
+        }();
     }
     float wv[W], bias_v;
     channel_taps<W>(p.weight, p.bias, p.w_dtype, p.w_stride_c, p.w_stride_w, c, wv, bias_v);

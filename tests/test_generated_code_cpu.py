@@ -38,3 +38,12 @@ def test_decode_of_a_few_tokens_keeps_eight_waves(tmp_path):
     text = _assembly("cc1d_update.hip", tmp_path)
     counts = re.findall(r"\.name:\s+\S*update_tokens_kernel\S*.*?\.vgpr_count:\s+(\d+)", text, re.S)
     assert counts and all(int(n) <= 64 for n in counts), counts
+
+
+def test_short_rows_ask_for_their_elements_at_once(tmp_path):
+    """Channel-first forward, rows shorter than a vector: a lane's up to 4 (16-bit: 8) elements are its first loads, and none is
+    waited for in front of the last."""
+    for name, body in _kernels(_assembly("cc1d_fwd_channelfirst.hip", tmp_path), "fwd_channelfirst_short_kernelILi[0-2]ELi[2-4]ELb[01]ELi2E"):
+        parts = body.split("global_load_")
+        elements = 4 if "kernelILi0E" in name else 8
+        assert not any("vmcnt" in part for part in parts[1:elements]), name
