@@ -384,9 +384,16 @@ int launch_taps(const FwdClArgs &a, const FwdClRare &q, int width, bool silu, in
 // (2, 352, 6320) 7.05 / 6.68 (593), fp32 (13, 3776, 40) with seq_idx 6.33 / 5.68 (576).  In between 16 rows are as fast ((1, 672, 4976) 5.37 /
 // 5.41 (467), fp32 (2, 1088, 907) 5.44 / 5.63 (485)), from 640 workgroups on faster ((1, 2152, 1208) fp32 6.79 / 7.35 (646)).  70
 // shapes of every type and alignment in these two ranges: 5 % on average, none slower than 0.3 %.
-static int choose_rows_per_run(int seqlen, int64_t row_bytes, int width, int64_t waves_at_default) {
+// Taps that are not packed (strided, or of another 16-bit type) are read one by one, which a run twice as short does
+// twice as often: up to 1536 wavefronts 8 rows are 2 to 11 % faster there too, but 16-bit ones 3 % slower at 1537 .. 1600, 2 % at
+// 2049 .. 2500 and up to 29 %, bf16 (8, 2536, 193) with strided taps 7.7 / 10.0 us (520 workgroups).
+static int choose_rows_per_run(int seqlen, int64_t row_bytes, int width, int64_t waves_at_default, bool packed_taps) {
     int T = tunables().fwd_cl_rows;
-    if (T <= 0) T = waves_at_default <= 1600 || (waves_at_default > 2048 && waves_at_default <= 2500) ? kGroup : kDefaultRows;
+    if (T <= 0) {
+        const bool eight = waves_at_default <= 1536 ||
+                           (packed_taps && (waves_at_default <= 1600 || (waves_at_default > 2048 && waves_at_default <= 2500)));
+        T = eight ? kGroup : kDefaultRows;
+    }
     const int cap = (seqlen + kGroup - 1) / kGroup * kGroup;      // never longer than the sequence
     if (T > cap) T = cap;
     T = (T + kGroup - 1) / kGroup * kGroup;
@@ -409,7 +416,7 @@ int launch_fwd_channellast(const cc1d_fwd_params &p, const cc1d_varlen_params *g
     const int64_t row_stride = p.x_stride_l > p.out_stride_l ? p.x_stride_l : p.out_stride_l;
     a.waves_per_row = (uint32_t)((a.n_cols + kWave - 1) / kWave);
     a.rows_per_run = choose_rows_per_run(p.seqlen, row_stride * eb, p.width,
-                                         (int64_t)p.batch * ((p.seqlen + kDefaultRows - 1) / kDefaultRows) * a.waves_per_row);
+                                         (int64_t)p.batch * ((p.seqlen + kDefaultRows - 1) / kDefaultRows) * a.waves_per_row, mode != 0);
     if (a.rows_per_run == 0) return CC1D_ERR_TOO_LARGE;
     a.n_runs = (p.seqlen + a.rows_per_run - 1) / a.rows_per_run;
     const int64_t total = (int64_t)p.batch * a.n_runs * a.waves_per_row;
