@@ -40,8 +40,11 @@ constexpr int kRsrcRaw = 0x00020000;              // buffer resource word 3: raw
 
 typedef void __attribute__((address_space(3))) *lds_ptr_t;
 
-// 184 bytes, three cache lines: with 200 the strides of final_states lay on a fourth cache line, which the wavefront asked for only when
-// everything else was done, 4 % of a launch of a few rows ((2, 20, 1536) fp16 with states 3.92 -> 4.10 us).
+// 192 bytes, three cache lines: with 200 the strides of final_states lay on a fourth, which the wavefront asked for only when everything
+// else was done, 4 % of a launch of a few rows ((2, 20, 1536) fp16 with states 4.08 / 3.85 us).  Whole words: with the small numbers as
+// bytes the compiler waited for all arguments to take batch_inner out of its word in front of the row's number, 0.5 % of large
+// launches ((4, 6704, 4288) bf16 with states 83.9 / 83.5 us, (16, 4096, 1001) 51.0 / 50.8).
+enum FwdCfTileStates : int { kHasInit = 0x100, kHasFinal = 0x200 };
 struct FwdCfTileArgs {
     uint32_t total;               // rows * tiles_per_row wavefronts
     uint32_t tiles_per_row;
@@ -49,10 +52,9 @@ struct FwdCfTileArgs {
     int32_t seqlen;
     int32_t body_vecs;            // vectors of a row that are walked as vectors (all of them, or a whole number of steps)
     uint32_t inner;               // what rows are numbered by: batch or dim
-    int8_t tail_vecs;             // vectors behind the body, done one position per lane (0: none)
-    int8_t batch_inner;           // rows numbered with the batch entry fastest
-    int8_t w_dtype;
-    int8_t states;                // bit 0: initial_states given, bit 1: final_states wanted
+    int32_t tail_vecs;            // vectors behind the body, done one position per lane (0: none)
+    int32_t batch_inner;          // rows numbered with the batch entry fastest
+    int32_t types;                // w_dtype, and kHasInit and kHasFinal where there are such states
     const void *x;
     void *out;
     const void *weight;
@@ -128,7 +130,7 @@ fwd_channelfirst_tile_kernel(const FwdCfTileArgs a) {
     T init_raw[W - 1];
 #pragma unroll
     for (int i = 0; i < W - 1; ++i) init_raw[i] = T(0.f);
-    if ((a.states & 1) != 0 && first_lane_of_row) {
+    if ((a.types & kHasInit) != 0 && first_lane_of_row) {
 #pragma unroll
         for (int i = 0; i < W - 1; ++i)
             init_raw[i] = ld_raw<DT>(a.initial_states, (int64_t)b * a.init_stride_b + (int64_t)c * a.init_stride_c +
@@ -138,7 +140,7 @@ fwd_channelfirst_tile_kernel(const FwdCfTileArgs a) {
     // (16, 4096, 1001) bf16 49.7 us against 47.3 with fp32 taps, 63.0 against 50.3 with bf16 taps;
     // (8, 5376, 2048) bf16 with bf16 taps 73.3 against 57.5.
     float wv_[W], bias_v;
-    uniform_taps<W>(a.weight, a.bias, a.w_dtype, a.w_stride_c, a.w_stride_w, c, wv_, bias_v);
+    uniform_taps<W>(a.weight, a.bias, a.types & 0xff, a.w_stride_c, a.w_stride_w, c, wv_, bias_v);
     if (SCALED) {
         bias_v *= kSiluPrescale;
 #pragma unroll
@@ -201,7 +203,7 @@ fwd_channelfirst_tile_kernel(const FwdCfTileArgs a) {
     // one that read initial_states: the two may be one buffer, and inside one wavefront the
     // reads are complete (the wait above) before the stores.  Rows here hold more than 64
     // vectors, so the values all come from x.
-    if ((a.states & 2) != 0 && tile == 0 && lane < W - 1) {
+    if ((a.types & kHasFinal) != 0 && tile == 0 && lane < W - 1) {
         const T v = ld_raw<DT>(xrow, L - (W - 1) + lane);
         st_raw<DT>(a.final_states, (int64_t)b * a.final_stride_b + (int64_t)c * a.final_stride_c +
                                        (int64_t)lane * a.final_stride_l, v);
@@ -283,8 +285,7 @@ int launch_fwd_channelfirst_tile(const cc1d_fwd_params &p, hipStream_t stream) {
     a.by_tiles = fast_div(a.tiles_per_row);
     a.inner = (uint32_t)(a.batch_inner ? p.batch : p.dim);
     a.by_inner = fast_div(a.inner);
-    a.w_dtype = (int8_t)p.w_dtype;
-    a.states = (int8_t)((p.initial_states != nullptr ? 1 : 0) | (p.final_states != nullptr ? 2 : 0));
+    a.types = p.w_dtype | (p.initial_states != nullptr ? kHasInit : 0) | (p.final_states != nullptr ? kHasFinal : 0);
     a.x = p.x; a.out = p.out; a.weight = p.weight; a.bias = p.bias;
     a.x_stride_b = p.x_stride_b; a.x_stride_c = p.x_stride_c;
     a.out_stride_b = p.out_stride_b; a.out_stride_c = p.out_stride_c;
